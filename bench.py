@@ -240,7 +240,7 @@ def batched_leg(st, ctx, batches, steps, warmup, seed):
                                        "busy cycles (SQ_VALU_MFMA_BUSY_CYCLES) in "
                                        "profiles/matmul_kernel_ffn_b8_b32.md",
                     "bytes_per_pass": nbytes,
-                    "kernel": "matmul_kernel + matmul_finish_kernel (matmul plan)",
+                    "kernel": "matmul_kernel (matmul plan)",
                     "launches_per_pass": 1,
                     "per_site_launches": {"launches_per_pass": len(sites),
                                           "ms_per_pass": round(ms_site, 4),

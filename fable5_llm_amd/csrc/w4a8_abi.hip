@@ -878,10 +878,6 @@ struct w4a8_mplan {
   void *d_table = nullptr;
   MmPlanCfg cfg{};
   bool built = false;
-  uint8_t *d_part = nullptr;  // the K-split jobs' slice sums
-  void *d_fin = nullptr;      // their finishing records
-  int nfin = 0;
-  int64_t fin_max = 0;        // the largest B * nrows among them
   // buffers of earlier builds: a graph the caller captured from an earlier
   // run still points at them, so they are freed only by destroy
   std::vector<void *> retired;
@@ -920,50 +916,22 @@ int w4a8_mplan_run(w4a8_mplan *p) {
     if (cs != hipStreamCaptureStatusNone)
       return fail(W4A8_E_ARG, "matmul plan: run it once before capturing it (the first "
                               "run after an add writes its device table)");
-    std::vector<uint8_t> host(matmul_job_bytes() * (size_t)n);
-    std::vector<int32_t> ns(n);
-    HIP_TRY(matmul_plan_prepare(p->jobs.data(), n, p->B, host.data(), &p->cfg, ns.data()));
-    for (void *q : {(void *)p->d_table, (void *)p->d_part, p->d_fin})
-      if (q) p->retired.push_back(q);
-    p->d_table = p->d_fin = nullptr;
-    p->d_part = nullptr;
-    // a K-split job's slices store their sums to part [ns][B][nrows] int64
-    std::vector<size_t> off(n, 0);
-    size_t part = 0;
-    for (int j = 0; j < n; ++j) {
-      if (ns[j] <= 1) continue;
-      off[j] = part;
-      part += ((size_t)ns[j] * p->B * (size_t)p->jobs[j].nrows * 8 + 255) & ~(size_t)255;
-    }
-    p->nfin = 0;
-    p->fin_max = 0;
-    if (part) {
-      HIP_TRY(hipMalloc(&p->d_part, part));
-      for (int j = 0; j < n; ++j) {
-        if (ns[j] <= 1) continue;
-        matmul_plan_bind(host.data(), j, (int64_t *)(p->d_part + off[j]));
-        const int64_t e = (int64_t)p->B * p->jobs[j].nrows;
-        p->fin_max = e > p->fin_max ? e : p->fin_max;
-      }
-      std::vector<uint8_t> fin(matmul_finish_bytes() * (size_t)n);
-      p->nfin = matmul_finish_prepare(host.data(), n, p->B, fin.data());
-      HIP_TRY(hipMalloc(&p->d_fin, fin.size()));
-      HIP_TRY(hipMemcpy(p->d_fin, fin.data(), fin.size(), hipMemcpyHostToDevice));
-    }
+    std::vector<uint8_t> host;
+    HIP_TRY(matmul_plan_prepare(p->jobs.data(), n, p->B, host, &p->cfg));
+    if (p->d_table) p->retired.push_back(p->d_table);
+    p->d_table = nullptr;
     HIP_TRY(hipMalloc(&p->d_table, host.size()));
     HIP_TRY(hipMemcpy(p->d_table, host.data(), host.size(), hipMemcpyHostToDevice));
     p->built = true;
   }
-  HIP_TRY(launch_matmul_plan(p->d_table, n, p->cfg, c->d_err, c->stream));
-  HIP_TRY(launch_matmul_finish(p->d_fin, p->nfin, p->fin_max, c->d_err, c->stream));
+  HIP_TRY(launch_matmul_plan(p->d_table, p->cfg, c->d_err, c->stream));
   return W4A8_OK;
 }
 
 int w4a8_mplan_destroy(w4a8_mplan *p) {
   if (!p) return W4A8_OK;
   int rc = W4A8_OK;
-  for (void *q : {(void *)p->d_table, (void *)p->d_part, p->d_fin})
-    if (q) p->retired.push_back(q);
+  if (p->d_table) p->retired.push_back(p->d_table);
   if (!p->retired.empty()) {
     DeviceGuard g(p->ctx->device);
     bool ok = hipStreamSynchronize(p->ctx->stream) == hipSuccess;

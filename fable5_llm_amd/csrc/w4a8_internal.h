@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 namespace w4a8 {
 
 // ---------------------------------------------------------------------------
@@ -275,30 +277,16 @@ struct MmJobSpec {
 hipError_t launch_matmul_multi(const MmJobSpec *jobs, int n, int32_t B, int32_t *err,
                                hipStream_t s);
 // A matmul plan: up to kMmPlanJobs matrices for the same B tokens in one
-// launch, their records in a device table (matmul_job_bytes() each) that
+// launch, their units of row tiles in a device table that
 // matmul_plan_prepare writes on the host, with the launch shape in cfg.
 constexpr int kMmPlanJobs = 128;
 struct MmPlanCfg {
-  int32_t B, CT, G, tmx, ctxt, R, nl, slot_bytes;
-  size_t lds;
+  int32_t B, CT, TM, KS, units, wgs;
 };
-size_t matmul_job_bytes();
-// ns[j] (out): job j's K slices; a job with ns[j] > 1 needs its reduction
-// buffers (zero) bound to its record before the first launch
-hipError_t matmul_plan_prepare(const MmJobSpec *jobs, int n, int32_t B, void *table,
-                               MmPlanCfg *cfg, int32_t *ns);
-// part: int64 [ns][B][nrows], the slices' sums (overwritten by every launch)
-void matmul_plan_bind(void *table, int j, int64_t *part);
-// The split jobs' finishing records (matmul_finish_bytes() each, at most n)
-// from a bound table; returns their count.  launch_matmul_finish, after each
-// launch of the plan, adds the slices and stores y32 (max_n: the largest
-// B * nrows among them).
-size_t matmul_finish_bytes();
-int matmul_finish_prepare(const void *table, int n, int32_t B, void *fin);
-hipError_t launch_matmul_finish(const void *d_fin, int nf, int64_t max_n, int32_t *err,
-                                hipStream_t s);
-hipError_t launch_matmul_plan(const void *d_table, int n, const MmPlanCfg &cfg,
-                              int32_t *err, hipStream_t s);
+hipError_t matmul_plan_prepare(const MmJobSpec *jobs, int n, int32_t B,
+                               std::vector<uint8_t> &table, MmPlanCfg *cfg);
+hipError_t launch_matmul_plan(const void *d_table, const MmPlanCfg &cfg, int32_t *err,
+                              hipStream_t s);
 hipError_t launch_matmul(const uint8_t *w, int32_t nrows, const Layout &L,
                          int32_t sh, const int8_t *x8, int32_t B,
                          int32_t *y32, int32_t *err, hipStream_t s);

@@ -1,44 +1,48 @@
 // Batched W4A8 (several tokens): int8 MFMA on gfx950 with the per-group
 // scale applied after accumulation.  Per token the result is bit-identical
 // to ref/w4a8_ref.py:254-289 matvec_y32: every group sum is exact in int32
-// (|16 * sum w*x| <= 2^21) and the scale products are summed exactly (in
-// int64 or, below 2^53, in double precision).
+// (|16 * sum w*x| <= 2^21) and the scale products are summed in int64.
 //
-// v_mfma_i32_16x16x64_i8: A = 16 weight rows x 64 k, B = 64 k x 16 tokens,
-// D = 16 x 16 int32.  Lane l feeds row/token (l % 16) and k-quarter l / 16
+// v_mfma_i32_16x16x64_i8: A = 16 tokens x 64 k, B = 64 k x 16 weight rows,
+// D = 16 x 16 int32.  Lane l feeds token / row (l % 16) and k-quarter l / 16
 // of A and B alike, so A and B share one lane->k mapping and the dot product
 // does not depend on the order in which the hardware walks k.  D element
-// (4 * (l / 16) + r, l % 16) lands in lane l, register r.
+// (4 * (l / 16) + r, l % 16) lands in lane l, register r: a lane holds four
+// tokens of ONE weight row, so a group's scale is one value per lane, read
+// from that row's own bytes of the scale block.  It enters through
+// v_mad_i64_i32, which runs at the rate of a double-precision FMA (measured:
+// 2.4 against 2.2 ns per instruction and SIMD) and needs no conversion.
 //
-// One workgroup per CU, 12 wavefronts:
+// Four wavefronts per workgroup, two workgroups per CU.  What bounds it is the
+// weight stream, and next to it the activations: 16 tokens of a group are
+// 2 KiB for every KiB of weights they meet.  Loaded straight into the MFMA's
+// layout they touch 16 cache lines per 16 lanes, and the address unit takes
+// one line a cycle; so they are copied into LDS in whole lines (8 tokens x 128
+// bytes a copy), with the 16-byte pieces of token t stored at piece ^ (t % 8),
+// which keeps the LDS reads free of bank conflicts.  Two ways to split a
+// unit (up to TM tiles per wavefront, all of K) over the wavefronts:
 //
-//  * 8 group wavefronts.  A tile's scale block b covers groups 8b..8b+7;
-//    wavefront w takes group 8b + w of every block, so the 8 read one
-//    block's 8 KiB of weights together.  Each keeps its next kMD 16-byte
-//    weight pieces in flight (uniform buffer loads: the compiler's count of
-//    its outstanding loads is exact, and a wait is for the oldest piece
-//    only).
-//  * up to 3 loader wavefronts copy, with LDS DMA, each block's activations
-//    (B tokens x 1 KiB) and the scale rows of the round's tiles into a ring
-//    of LDS slots, ahead of the group wavefronts, and flag each slot once its
-//    copies have landed.
-//  * 1 store wavefront: at the end of a round the 8 group wavefronts add
-//    their sums into an LDS table (two tables, alternating by round);
-//    the store wavefront rounds, checks and stores the round's y32 and frees
-//    the table.  Group wavefronts thus issue no stores, which would make the
-//    compiler's count of their outstanding loads unknown.
+//  * shared (KS = 1): every wavefront takes its own TM tiles and all of K, and
+//    the four share one copy of the activations (one workgroup barrier per
+//    four groups).  Nothing is reduced; best where tiles are plenty.
+//  * split (KS = 4): the wavefronts take the same tile and every fourth quad
+//    of groups, each with its own copies (no barrier), and meet in an LDS
+//    table at the end of the unit.
 //
-// A workgroup works through its tiles in rounds of up to TM tiles (TM * CT
-// <= 4, CT = column tiles of 16 tokens), block-major within a round, so that
-// each block's activations serve every tile of the round.  One launch may
-// carry several matrices (jobs, same tokens, each its own activations): a
-// workgroup's rounds run through its tiles of job 0, then job 1, ..., and
-// the ring, the loaders and the weight pieces in flight run on across the
-// job boundaries, so the weight stream does not drain between matrices.  Every wait between wavefronts is bounded: a wait that gives
-// up sets bit 2 of the error word and an abort word, after which no wait of
-// the workgroup polls again, so a launch always drains.
-#include <type_traits>
-#include <vector>
+// A workgroup runs its units one after another; the weight ring (4 groups per
+// wavefront) and the copies run on across them, so the stream does not drain
+// between tiles or matrices.  No wait depends on another workgroup.
+//
+// Measured, cold weights (us per launch, before: one workgroup per CU with
+// loader wavefronts and 8 slots, which waited for each slot's copies in turn):
+//   12288 + 12288 rows, K 4096:  B = 8: 19.0 -> 14.0, B = 64: 100 -> 21
+//   4096 rows, K 12288:          B = 8: 12.8 -> 10.2, B = 64: 52 -> 19
+//   60,000 rows, K 4096:         B = 8: 32 -> 25, B = 32: 50 -> 30, B = 64: 241 -> 40
+//   a pass of 96 FFN matrices:   B = 8: 534 -> 464, B = 32: 711 -> 565, B = 64: 4040 -> 680
+// (the pass's weights alone take 360 us at the read ceiling).  The 117 MB
+// of y32 that a pass writes at B = 32 cost 55 us of it (a copy that stores
+// nothing), the rest is the activations' way through L1 and LDS.
+#include <algorithm>
 
 #include "w4a8_device.h"
 
@@ -48,76 +52,38 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-constexpr int kMW = 8;                     // group wavefronts 0..7
-constexpr int kML = 3;                     // loader wavefronts 8..10 (at most)
-constexpr int kMStore = kMW + kML;         // the store wavefront, 11
-constexpr int kMThreads = (kMW + kML + 1) * 64;
-constexpr int kXRow = 1024 + 16;           // LDS bytes per token of a block's activations
 constexpr int kMBufDword3 = 0x00020000;    // raw buffer, 32-bit data format
 constexpr int kMAuxNt = 2;                 // buffer-load cache policy: non-temporal
-constexpr int kRingMax = 8;
+constexpr int kMPast = 0x40000000;         // a buffer offset past every range
 constexpr int kLdsBytes = 160 * 1024;
+constexpr int kMWaves = 4;
+constexpr int kMThreads = 64 * kMWaves;
 
-static_assert(kXRow % 16 == 0, "token rows stay 16-byte aligned");
-
-struct MmJob {
-  const uint8_t *W;     // tile layout
+// A unit: up to TM * TS consecutive row tiles of one matrix, over all of K.
+struct MmUnit {
+  const uint8_t *W;     // first tile
   const int8_t *x8;     // [B][K]
   int32_t *y32;         // [B][nrows]
-  int64_t tile_bytes;
-  int32_t nrows, ntiles, NG, nblk, sh, K;
-  int32_t tm;           // tiles per round
-  int32_t ns;           // K slices (1: none), see the split below
-  int64_t *part;        // split: [ns][B][nrows] each slice's sums (16 p)
+  int32_t tile_bytes, ntiles;   // tiles from W on
+  int32_t nrows, row0;  // row0: the first tile's first row
+  int32_t NG, K, sh;
+  int32_t pad[3];
 };
+static_assert(sizeof(MmUnit) == 64, "one scalar load of 16 words");
 
-// A split job (ns > 1; a matrix with at most one tile per workgroup) cuts
-// K into ns slices of nblk / ns blocks.  Workgroup r takes slice r % ns of
-// row tiles r / ns, r / ns + G / ns, ...: its rounds' tiles share one copy
-// of the slice's activations, and a workgroup reads only its slice, the
-// same one on every workgroup of its XCD (r % 8, with ns dividing 8).  Each
-// slice stores its sums to part; matmul_finish_kernel adds the ns slices,
-// rounds, checks and stores y32 after the launch.
-struct MmSlice {
-  int tr, tg, kb0, nbs;   // first row tile, row-tile stride, first block, blocks
-  // ns is 1, 2 or 4 (the host's choice), so the divisions are shifts
-  __device__ MmSlice(const MmJob &J, int r, int G) {
-    const int l = __builtin_ctz((unsigned)J.ns);
-    tr = r >> l;
-    tg = G >> l;
-    nbs = J.nblk >> l;
-    kb0 = (r & (J.ns - 1)) * nbs;
-  }
+struct MmJob {
+  MmUnit u;             // the job's first unit
+  int32_t unit0;        // its number
+  int32_t pad[3];
 };
 
 struct MmParams {
   MmJob job[kMmJobs];   // the jobs, when they travel in the parameters ...
-  const MmJob *tab;     // ... or a device table of njobs (a matmul plan)
-  int32_t njobs;
-  int32_t B, CT;
-  int32_t R;            // LDS slots
-  int32_t nl;           // loader wavefronts in use
-  int32_t slot_bytes;   // 16 * CT token rows of kXRow, then tm scale rows of 256 B
+  const MmUnit *tab;    // ... or a device table of the units (a matmul plan)
+  int32_t njobs, units;
+  int32_t B;
   int32_t *err;
 };
-
-// LDS: flags, then the reduction tables, then the ring of slots
-struct MmFlags {
-  int32_t ready[kRingMax];   // step whose copies have landed in the slot (-1: none)
-  int32_t done[kMW];         // last step each group wavefront has finished (-1: none)
-  int32_t tgen[2];           // round allowed to add into each table next
-  int32_t tcnt[2];           // group wavefronts that have added this round
-  int32_t abort;
-  int32_t err;
-  int32_t pad[2];
-  // this workgroup's schedule: job j has nmine[j] of its tiles, global
-  // rounds rbase[j] .. rbase[j + 1] - 1 and steps sbase[j] .. sbase[j + 1] - 1
-  int32_t nmine[kMmPlanJobs];
-  int32_t rbase[kMmPlanJobs + 1];
-  int32_t sbase[kMmPlanJobs + 1];
-};
-static_assert(kMmPlanJobs <= 128, "the schedule scan takes two jobs a lane");
-constexpr int kFlagBytes = (int)((sizeof(MmFlags) + 255) / 256 * 256);
 
 __device__ __forceinline__ int cvt_lo16(uint32_t w) {
   // offset-form low nibbles u = w + 8 -> bytes 16*w (exact int8)
@@ -127,730 +93,486 @@ __device__ __forceinline__ int cvt_hi16(uint32_t w) {
   return (int)(w & 0xF0F0F0F0u);   // two's-complement high nibbles -> 16*w
 }
 
-__device__ __forceinline__ int64_t rshr64_mm(int64_t v, int s) {
-  if (s == 0) return v;
-  const int64_t half = (int64_t)1 << (s - 1);
-  return v >= 0 ? ((v + half) >> s) : -((-v + half) >> s);
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const void *p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, bytes, kMBufDword3);
 }
 
-__device__ __forceinline__ void mm_wait_vm_all() {
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+// A group's activations, both 16-byte halves of a lane's 32 k for every tile
+// of 16 tokens (2 KiB apart).  In assembly, with the wait in the same block:
+// the compiler would make an LDS read wait for the newest LDS copy in flight.
+template <int CT>
+__device__ __forceinline__ void mm_read(v4i (&x)[CT][2], uint32_t o0, uint32_t o1) {
+  if constexpr (CT == 1) {
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(x[0][0]), "=&v"(x[0][1]) : "v"(o0), "v"(o1) : "memory");
+  } else if constexpr (CT == 2) {
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
+                 "ds_read_b128 %2, %4 offset:2048\n\tds_read_b128 %3, %5 offset:2048\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1])
+                 : "v"(o0), "v"(o1) : "memory");
+  } else if constexpr (CT == 3) {
+    asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %7\n\t"
+                 "ds_read_b128 %2, %6 offset:2048\n\tds_read_b128 %3, %7 offset:2048\n\t"
+                 "ds_read_b128 %4, %6 offset:4096\n\tds_read_b128 %5, %7 offset:4096\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1]),
+                   "=&v"(x[2][0]), "=&v"(x[2][1])
+                 : "v"(o0), "v"(o1) : "memory");
+  } else {
+    asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\t"
+                 "ds_read_b128 %2, %8 offset:2048\n\tds_read_b128 %3, %9 offset:2048\n\t"
+                 "ds_read_b128 %4, %8 offset:4096\n\tds_read_b128 %5, %9 offset:4096\n\t"
+                 "ds_read_b128 %6, %8 offset:6144\n\tds_read_b128 %7, %9 offset:6144\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1]),
+                   "=&v"(x[2][0]), "=&v"(x[2][1]), "=&v"(x[3][0]), "=&v"(x[3][1])
+                 : "v"(o0), "v"(o1) : "memory");
+  }
 }
-__device__ __forceinline__ void mm_lds_add(double *p, double v) {
-  asm volatile("ds_add_f64 %0, %1" :: "v"(lds_off(p)), "v"(v) : "memory");
+
+__device__ __forceinline__ int32_t mm_opaque(int32_t v) {
+  asm("" : "+v"(v));
+  return v;
 }
 __device__ __forceinline__ void mm_lds_add(int64_t *p, int64_t v) {
   asm volatile("ds_add_u64 %0, %1" :: "v"(lds_off(p)), "v"(v) : "memory");
 }
-
-// The sums of scale x group products of a kernel instance: exact either
-// way (every product < 2^16 * 2^21, every partial sum < 96 groups * 2^37 <
-// 2^44: integers below 2^53), in double precision (full-rate FMAs) where two
-// or more column tiles give each scale several products, else in int64
-// (quarter-rate multiply-adds, but no conversions)
-template <int CTX>
-using MmAcc = typename std::conditional<(CTX >= 2), double, int64_t>::type;
-template <int CTX>
-__device__ __forceinline__ MmAcc<CTX> mm_scale(int32_t m) { return (MmAcc<CTX>)m; }
-__device__ __forceinline__ double mm_fma(double m, int32_t a, double p) {
-  return __builtin_fma(m, (double)a, p);
-}
-__device__ __forceinline__ int64_t mm_fma(int64_t m, int32_t a, int64_t p) {
-  return p + m * (int64_t)a;
-}
-__device__ __forceinline__ int32_t mm_lds_add_rtn(int32_t *p, int32_t v) {
-  int32_t old;
-  asm volatile("s_waitcnt lgkmcnt(0)\n\tds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)"
-               : "=v"(old) : "v"(lds_off(p)), "v"(v) : "memory");
-  return old;
-}
-// an LDS add that does not wait for itself (nor for earlier LDS work)
-__device__ __forceinline__ void mm_lds_add_post(int32_t *p, int32_t v) {
-  asm volatile("ds_add_u32 %0, %1" :: "v"(lds_off(p)), "v"(v) : "memory");
-}
-// an LDS write that does not wait for itself (nor for earlier LDS work: a
-// wavefront's LDS instructions execute in order)
-__device__ __forceinline__ void mm_lds_post(int32_t *p, int32_t v) {
-  asm volatile("ds_write_b32 %0, %1" :: "v"(lds_off(p)), "v"(v) : "memory");
-}
-__device__ __forceinline__ void mm_lds_or(int32_t *p, int32_t v) {
-  asm volatile("ds_or_b32 %0, %1" :: "v"(lds_off(p)), "v"(v) : "memory");
-}
-// lane l copies 16 (or 4) bytes from its own address to LDS lds_base + 16 l
-// (4 l); lds_base must be uniform
-__device__ __forceinline__ void dma16(const void *src, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
-               :: "v"(src), "s"(lds_base) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(const void *src, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off"
-               :: "v"(src), "s"(lds_base) : "memory", "m0");
+// the entry's value, the entry cleared
+__device__ __forceinline__ int64_t mm_lds_take(int64_t *p) {
+  int64_t v;
+  asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)\n\tds_write_b64 %1, %2"
+               : "=&v"(v) : "v"(lds_off(p)), "v"((int64_t)0) : "memory");
+  return v;
 }
 
-// Bounded LDS wait of one wavefront: until every lane's predicate holds,
-// the workgroup aborts, or kLdsSpin polls (then bit 2 of err and abort).
-template <typename Pred>
-__device__ __forceinline__ bool mm_wait(MmFlags &F, Pred pred) {
-  for (uint32_t n = 0;; ++n) {
-    if (__all(pred())) return true;
-    if (lds_read_i32(&F.abort) != 0) return false;
-    if (n > kLdsSpin) {
-      if ((threadIdx.x & 63) == 0) {
-        lds_write_i32(&F.abort, 1);
-        mm_lds_or(&F.err, 4);
-      }
-      return false;
-    }
-    __builtin_amdgcn_s_sleep(1);
-  }
+// s_waitcnt vmcnt(N) alone (gfx9 encoding: vmcnt in bits 3:0 and 15:14)
+template <int N>
+__device__ __forceinline__ void mm_wait_vm() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
 }
 
-// The same wait for a group wavefront, as a loop of plain exits (the form
-// in which the compiler keeps its count of outstanding weight loads across
-// it): until the LDS word at p is at least v (kAtLeast) or equal to v.
-template <bool kAtLeast>
-__device__ __forceinline__ void mm_wait_word(MmFlags &F, const int32_t *p, int v, int lane) {
-  for (uint32_t n = 0;; ++n) {
-    const int32_t cur = lds_read_i32(p);
-    if (__all(kAtLeast ? cur >= v : cur == v)) break;
-    if (lds_read_i32(&F.abort) != 0) break;
-    if (n > kLdsSpin) {
-      if (lane == 0) {
-        lds_write_i32(&F.abort, 1);
-        mm_lds_or(&F.err, 4);
-      }
-      break;
-    }
-    __builtin_amdgcn_s_sleep(1);
-  }
-}
-
-// A workgroup's tiles of a job are r, r + G, ...; the job's round rho takes
-// tiles rho*tm .. rho*tm + nt - 1 of them, and the job's step
-// rho * nblk + kb covers block kb of every tile of round rho.
-__device__ __forceinline__ int round_tiles(const MmJob &J, int nmine, int rho) {
-  return min(J.tm, nmine - rho * J.tm);
-}
-
-// Position in this workgroup's schedule: job j, its round rho and block kb;
-// RHO counts rounds over all jobs.  Jobs with no tile on this workgroup are
-// skipped.  The fields of job j that a step needs stay in registers, so the
-// job table and the schedule in LDS are read only when the job changes (a
-// read on every step puts its latency on every step).
-struct MmCur {
-  int j, rho, kb, RHO;     // kb: block of the slice (kb0 + kb of the matrix)
-  int rend;                // first round past job j
-  int nblk, tm, nmine, nt, NG, K;
-  int tr, tg, kb0;         // the workgroup's slice (MmSlice; nblk = its blocks)
-  const uint8_t *W;
-  const int8_t *x8;
-  int64_t tile_bytes;
-  template <class JobF>
-  __device__ void load(const MmFlags &F, int njobs, JobF &JOB) {
-    if (j >= njobs) return;
-    const MmJob &J = JOB(j);
-    const MmSlice S(J, (int)blockIdx.x, (int)gridDim.x);
-    tr = S.tr;
-    tg = S.tg;
-    kb0 = S.kb0;
-    nblk = S.nbs;
-    tm = J.tm;
-    NG = J.NG;
-    K = J.K;
-    W = J.W;
-    x8 = J.x8;
-    tile_bytes = J.tile_bytes;
-    nmine = __builtin_amdgcn_readfirstlane(F.nmine[j]);
-    rend = __builtin_amdgcn_readfirstlane(F.rbase[j + 1]);
-    nt = min(tm, nmine - rho * tm);
-  }
-  template <class JobF>
-  __device__ void start(const MmFlags &F, int njobs, JobF &JOB) {
-    j = 0;
-    rho = kb = RHO = 0;
-    nt = 0;
-    W = nullptr;
-    while (j < njobs && F.rbase[j + 1] == 0) ++j;
-    load(F, njobs, JOB);
-  }
-  template <class JobF>
-  __device__ void next(const MmFlags &F, int njobs, JobF &JOB) {
-    if (++kb < nblk) return;
-    kb = 0;
-    ++rho;
-    ++RHO;
-    if (RHO < rend) {
-      nt = min(tm, nmine - rho * tm);
-      return;
-    }
-    rho = 0;
-    while (j < njobs && RHO == F.rbase[j + 1]) ++j;
-    load(F, njobs, JOB);
-  }
+struct MmSrc {
+  const uint8_t *w;
+  const int8_t *x;
+  int32_t tile_bytes, ntiles, K, NG;
 };
-
-// Put group 8 kb + w of tile j of the cursor's round in flight: a buffer
-// load whose range is empty (no memory access, zeros) when there is no such
-// tile or group, so every step issues the same loads.
-__device__ __forceinline__ uint4 mm_issue(const MmCur &C, int r, int G, int w, int lane, int j,
-                                          bool real) {
-  const uint8_t *base = C.W;
-  int len = 0;
-  const int kb = C.kb0 + C.kb;
-  if (real && 8 * kb + w < C.NG) {
-    const int64_t t = (int64_t)C.tr + (int64_t)C.tg * (C.rho * C.tm + j);
-    base = C.W + t * C.tile_bytes + (int64_t)kb * kBlockBytes + kScaleChunk +
-           (int64_t)w * kGroupChunk;
-    len = kGroupChunk;
-  }
-  const __amdgpu_buffer_rsrc_t rs =
-      __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, len, kMBufDword3);
-  // lane (c = l % 16, q = l / 16) takes row c's quarter q: bytes (4c + q) * 16
-  const int piece = ((lane & 15) * 4 + (lane >> 4)) * 16;
-  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-  const u4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, piece, 0, kMAuxNt);
-  return make_uint4(v.x, v.y, v.z, v.w);
+// tile j's buffer: its range ends with the tile's data, and is empty (loads
+// return zeros without a memory access) where there is no such tile
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_tile_rsrc(const MmSrc &S, int j) {
+  return mm_rsrc(S.w + (int64_t)j * S.tile_bytes, j < S.ntiles ? S.tile_bytes : 0);
 }
 
-// steps in flight per group wavefront: TMX pieces each (one tile a round,
-// as for a matrix with no more tiles than workgroups, goes 8 steps deep)
-template <int TMX, int CTX>
-constexpr int mm_depth() { return TMX >= 3 ? 4 : 8; }
+// A wavefront's step (the groups of one copy) and its LDS buffers: 4 groups
+// and two buffers where a buffer stays within 8 KiB per wavefront (32 KiB
+// shared), else one group and four buffers -- a step's copies are then
+// issued three groups ahead (17..32 tokens, 4096 rows, K 12288: 14.9 us with
+// two buffers, 13.8 with four).
+constexpr int mm_q(int CT, int KS) { return KS == 1 || CT == 1 ? 4 : 1; }
+constexpr int mm_nbuf(int CT, int KS) { return KS == 1 || CT == 1 ? 2 : 4; }
+constexpr int mm_octets(int CT, bool half8) { return half8 ? 1 : 2 * CT; }   // of tokens
+constexpr size_t mm_x_bytes(int CT, int KS, bool half8) {
+  return (size_t)KS * mm_nbuf(CT, KS) * mm_q(CT, KS) * mm_octets(CT, half8) * 1024;
+}
 
-template <int TMX, int CTX, bool kTab>
-__global__ __launch_bounds__(kMThreads) void matmul_kernel(MmParams P) {
-  extern __shared__ __align__(16) uint8_t smem[];
-  // job j (j uniform): from the parameters, or from the plan's device table
-  // read as constant memory, so that its fields come in by scalar loads and
-  // no wait for them counts the weight pieces in flight
-  typedef const __attribute__((address_space(4))) MmJob CJob;
-  auto JOB = [&](int j) -> const MmJob & {
-    const int ju = __builtin_amdgcn_readfirstlane(j);
-    if constexpr (kTab)
-      return *(const MmJob *)((CJob *)P.tab + ju);
-    else
-      return P.job[ju];
-  };
-  MmFlags &F = *(MmFlags *)smem;
-  typedef MmAcc<CTX> Acc;
-  Acc *tables = (Acc *)(smem + kFlagBytes);   // [2][TMX][CTX][4][64]
-  uint8_t *ring = smem + kFlagBytes + 2 * TMX * CTX * 4 * 64 * 8;
-  const int tid = threadIdx.x, lane = tid & 63;
+// half8: at most 8 tokens (one octet is copied, and read by both halves of
+// the MFMA's 16 rows)
+template <int TM, int CT, int KS, bool half8, bool plan>
+__global__ __launch_bounds__(kMThreads, 2) void matmul_kernel(MmParams P) {
+  extern __shared__ __align__(1024) uint8_t smem[];
+  constexpr int NW = kMWaves, TS = NW / KS;
+  constexpr int Q = mm_q(CT, KS), NBUF = mm_nbuf(CT, KS);
+  constexpr int NO = mm_octets(CT, half8);
+  constexpr int kGrp = NO * 1024;                   // LDS bytes of a group's activations
+  constexpr int kBuf = Q * kGrp;                    // ... of a step
+  constexpr int ND = TS == 1 ? Q * NO : Q * NO / NW;   // copies per wavefront and step
+  constexpr int D = 4;                              // groups in flight
+  constexpr int kTurn = KS * D;                     // groups of a turn of the ring, all slices
+  constexpr int kXBytes = (int)mm_x_bytes(CT, KS, half8);
+  constexpr int NR = TM * CT * 4 * 64;              // a wavefront's sums
+  static_assert(KS == 1 || KS == NW, "the copies are shared by all wavefronts or by none");
+  static_assert(ND * 1024 * (TS == 1 ? 1 : NW) == kBuf, "whole copies per wavefront");
+  static_assert(NBUF - 1 < D / Q || NBUF == 2, "a step's copies reach one turn ahead at most");
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int G = gridDim.x, r = blockIdx.x;
+  const int ks = TS == 1 ? wave : 0, ts = TS == 1 ? 0 : wave;
+  const int B = P.B, G = gridDim.x, r = blockIdx.x;
+  typedef const __attribute__((address_space(4))) MmUnit CUnit;
 
-  if (tid < kRingMax) F.ready[tid] = -1;
-  if (tid < kMW) F.done[tid] = -1;
-  if (tid < 2) {
-    F.tgen[tid] = tid;
-    F.tcnt[tid] = 0;
-  }
-  if (tid == 0) {
-    F.abort = 0;
-    F.err = 0;
-  }
-  // thread j: job j's tiles, rounds and steps on this workgroup ...
-  if (tid < P.njobs) {
-    const MmJob &J = kTab ? P.tab[tid] : P.job[tid];
-    const MmSlice S(J, r, G);
-    const int nm = S.tr < J.ntiles ? (J.ntiles - 1 - S.tr) / S.tg + 1 : 0;
-    const int nr = (nm + J.tm - 1) / J.tm;
-    F.nmine[tid] = nm;
-    F.rbase[tid + 1] = nr;
-    F.sbase[tid + 1] = nr * S.nbs;
-  }
-  for (int i = tid; i < 2 * TMX * CTX * 4 * 64; i += kMThreads) tables[i] = 0;
-  __syncthreads();
-  // ... and wavefront 0's prefix sums of them (lane l: jobs 2l, 2l + 1)
-  if (wave == 0) {
-    const int j0 = 2 * lane, j1 = 2 * lane + 1;
-    const int a0 = j0 < P.njobs ? F.rbase[j0 + 1] : 0, b0 = j0 < P.njobs ? F.sbase[j0 + 1] : 0;
-    const int a1 = j1 < P.njobs ? F.rbase[j1 + 1] : 0, b1 = j1 < P.njobs ? F.sbase[j1 + 1] : 0;
-    int sa = a0 + a1, sb = b0 + b1;
+  // unit number i of this workgroup (an empty one past its last)
+  auto unit_at = [&](int i) {
+    const int64_t pos = (int64_t)i * G + r;
+    MmUnit U{};
+    if constexpr (plan) {
+      if (pos < P.units) U = *(const MmUnit *)((CUnit *)P.tab + pos);
+    } else if (pos < P.units) {
+      const int u = (int)pos;
+      int jb = 0;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int ta = __shfl_up(sa, o), tb = __shfl_up(sb, o);
-      if (lane >= o) {
-        sa += ta;
-        sb += tb;
-      }
+      for (int k = 1; k < kMmJobs; ++k) jb += (k < P.njobs && u >= P.job[k].unit0) ? 1 : 0;
+      jb = __builtin_amdgcn_readfirstlane(jb);
+      U = P.job[jb].u;
+      const int t = (u - P.job[jb].unit0) * (TM * TS);
+      U.W += (int64_t)t * U.tile_bytes;
+      U.ntiles -= t;
+      U.row0 = t * kTileRows;
     }
-    const int ea = sa - a0 - a1, eb = sb - b0 - b1;   // before job j0
-    if (j0 < P.njobs) {
-      F.rbase[j0 + 1] = ea + a0;
-      F.sbase[j0 + 1] = eb + b0;
-    }
-    if (j1 < P.njobs) {
-      F.rbase[j1 + 1] = sa;
-      F.sbase[j1 + 1] = sb;
-    }
-    if (lane == 0) F.rbase[0] = F.sbase[0] = 0;
-  }
-  __syncthreads();
-  const int nrounds = F.rbase[P.njobs], nsteps = F.sbase[P.njobs];
+    return U;
+  };
+  // where a turn's loads come from
+  auto src_of = [&](const MmUnit &U) {
+    return MmSrc{U.W + (int64_t)(ts * TM) * U.tile_bytes, U.x8, U.tile_bytes, U.ntiles - ts * TM,
+                 U.K, U.NG};
+  };
 
-  if (wave == kMStore) {
-    // round rho's sums are complete once all 8 group wavefronts have added
-    bool ok = true;
-    int jb = 0;
-    for (int RHO = 0; RHO < nrounds; ++RHO) {
-      while (RHO >= F.rbase[jb + 1]) ++jb;   // rounds ascend: the job advances
-      const MmJob &J = JOB(jb);
-      const int rho = RHO - F.rbase[jb];
-      const int tb = RHO & 1, nt = round_tiles(J, F.nmine[jb], rho);
-      Acc *tbl = tables + tb * (TMX * CTX * 4 * 64);
-      if (!mm_wait(F, [&] { return lds_read_i32(&F.tcnt[tb]) == kMW; })) {
-        ok = false;
-        break;
-      }
-      const int q = lane >> 4, c = lane & 15;
-      // the job's fields, read once (kept in registers across the stores)
-      int32_t *const yj = J.y32;
-      const int32_t nrj = J.nrows, shj = J.sh, tmj = J.tm, nsj = J.ns;
-      const MmSlice S(J, r, G);
-      const int64_t half = shj > 0 ? (int64_t)1 << (shj - 1) : 0;
-      // every table entry read at once, then rounded, checked and stored
-      int64_t tot[TMX][CTX][4];
+  // a step's copies: 8 tokens of one group at a time (1 KiB): lane l brings
+  // piece (l % 8) ^ (token % 8) of token l / 8
+  const int dtok = lane >> 3, dpiece = (lane & 7) ^ (dtok & 7);
+  uint8_t *const xmine = smem + (TS == 1 ? wave * (NBUF * kBuf) : 0);
+  // the copies of a step whose first group (over all slices) is gs
+  auto copy_x = [&](const MmSrc &S, int gs, int buf) {
+    const __amdgpu_buffer_rsrc_t rx = mm_rsrc(S.x, B * S.K);
 #pragma unroll
-      for (int jj = 0; jj < TMX; ++jj)
-#pragma unroll
-        for (int ct = 0; ct < CTX; ++ct)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            tot[jj][ct][e] = (int64_t)tbl[((jj * CTX + ct) * 4 + e) * 64 + lane];
-#pragma unroll
-      for (int jj = 0; jj < TMX; ++jj)
-#pragma unroll
-        for (int ct = 0; ct < CTX; ++ct)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            tbl[((jj * CTX + ct) * 4 + e) * 64 + lane] = 0;
-      bool ovf = false;
-      // y = rshift_round(tot / 16, sh) (tot = 16 p): the magnitude rounded
-      // half up, checked and stored
-      auto put = [&](int64_t tt, int32_t *yp) {
-        const int64_t v = tt >> 4;
-        const int64_t m = ((v < 0 ? -v : v) + half) >> shj;
-        const int64_t y = v < 0 ? -m : m;
-        ovf = ovf || y > 2147483647LL || y < -2147483647LL;
-        *yp = (int32_t)y;
-      };
-      if (nsj == 1) {
-#pragma unroll
-        for (int ct = 0; ct < CTX; ++ct) {
-          const int tok = ct * 16 + c;
-          int32_t *const yt = yj + (int64_t)tok * nrj;
-#pragma unroll
-          for (int jj = 0; jj < TMX; ++jj) {
-            const int64_t row0 =
-                ((int64_t)S.tr + (int64_t)S.tg * (rho * tmj + jj)) * kTileRows + 4 * q;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (jj < nt && ct < P.CT && tok < P.B && row0 + e < nrj)
-                put(tot[jj][ct][e], yt + row0 + e);
-          }
-        }
-      } else {
-        // this slice's sums to its part of the job's partials, for
-        // matmul_finish_kernel
-        int64_t *const pj = J.part + (int64_t)(S.kb0 / S.nbs) * P.B * nrj;
-#pragma unroll
-        for (int ct = 0; ct < CTX; ++ct) {
-          const int tok = ct * 16 + c;
-#pragma unroll
-          for (int jj = 0; jj < TMX; ++jj) {
-            const int64_t row0 =
-                ((int64_t)S.tr + (int64_t)S.tg * (rho * tmj + jj)) * kTileRows + 4 * q;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (jj < nt && ct < P.CT && tok < P.B && row0 + e < nrj)
-                pj[(int64_t)tok * nrj + row0 + e] = tot[jj][ct][e];
-          }
-        }
-      }
-      if (ovf) mm_lds_or(&F.err, 1);
-      wait_lds();
-      if (lane == 0) {
-        lds_write_i32(&F.tcnt[tb], 0);
-        lds_write_i32(&F.tgen[tb], RHO + 2);
-      }
+    for (int d = 0; d < ND; ++d) {
+      const int n = TS == 1 ? d : wave * ND + d;    // (group, token octet)
+      const int g = n / NO, o = n % NO;
+      const int gg = gs + ks * D + g;
+      const int off = (8 * o + dtok) * S.K + gg * kGroup + 16 * dpiece;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rx, (lds_void_t *)(xmine + buf * kBuf + n * 1024), 16, gg < S.NG ? off : kMPast, 0, 0, 0);
     }
-    if (!ok && lane == 0) mm_lds_or(&F.err, 4);
-  } else if (wave >= kMW) {
-    // loader l: steps l, l + nl, ...
-    const int l = wave - kMW;
-    if (l < P.nl) {
-      MmCur lc;   // step s of this loader
-      lc.start(F, P.njobs, JOB);
-      for (int i = 0; i < l && i < nsteps; ++i) lc.next(F, P.njobs, JOB);
-      int slot = l;   // s % R (l < nl < R)
-      for (int s = l; s < nsteps; s += P.nl) {
-        // the slot's previous step has been consumed by every group wavefront
-        if (s >= P.R &&
-            !mm_wait(F, [&] { return lds_read_i32(&F.done[lane & (kMW - 1)]) >= s - P.R; }))
-          break;
-        uint8_t *sb = ring + (size_t)slot * P.slot_bytes;
-        const int kb = lc.kb0 + lc.kb;
-        const int kbytes = min(1024, lc.K - kb * 1024);   // multiple of 128
-        for (int tok = 0; tok < P.B; ++tok) {
-          const int8_t *src = 16 * lane < kbytes
-                                  ? lc.x8 + (int64_t)tok * lc.K + kb * 1024 + 16 * lane
-                                  : lc.x8;   // nothing to copy: any mapped address
-          dma16(src, lds_off(sb + tok * kXRow));
+  };
+  const int wlane = kScaleChunk + (c * 4 + q) * 16, slane = c * 16;
+  u4 w[TM][D];
+  uint32_t m[TM][D];
+  auto load_w = [&](const MmSrc &S, int g, const int slot) {
+    const int off = (g >> 3) * kBlockBytes + (g & 7) * kGroupChunk + wlane;
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+      w[j][slot] = __builtin_amdgcn_raw_buffer_load_b128(mm_tile_rsrc(S, j), off, 0, kMAuxNt);
+  };
+  auto load_m = [&](const MmSrc &S, int g, const int slot) {
+    const int off = (g >> 3) * kBlockBytes + (g & 7) * 2 + slane;
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+      m[j][slot] = __builtin_amdgcn_raw_buffer_load_b16(mm_tile_rsrc(S, j), off, 0, kMAuxNt);
+  };
+
+  int64_t p[TM][CT][4];
+#pragma unroll
+  for (int j = 0; j < TM; ++j)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p[j][ct][e] = 0;
+
+  MmUnit U = unit_at(0), V = unit_at(1);
+  MmSrc S = src_of(U);
+  int64_t *const red = (int64_t *)(smem + kXBytes);   // KS > 1: two tables of NR sums
+  if constexpr (KS > 1) {
+    for (int i = tid; i < 2 * NR; i += NW * 64) red[i] = 0;
+    wait_lds();
+    __builtin_amdgcn_s_barrier();
+  }
+#pragma unroll
+  for (int s = 0; s < NBUF - 1; ++s) copy_x(S, s / (D / Q) * kTurn + s % (D / Q) * Q, s);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < D; ++i) {
+    load_w(S, ks * D + i, i);
+    load_m(S, ks * D + i, i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // the first step's activations: everything issued after them may be in flight
+  mm_wait_vm<(NBUF - 2) * ND + 2 * TM * D>();
+  if constexpr (TS > 1) __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+
+  const int crow = half8 ? c & 7 : c;
+  const uint32_t xbase = lds_off(xmine) + crow * 128;
+  const uint32_t x0 = xbase + (((2 * q) ^ (c & 7)) * 16), x1 = xbase + (((2 * q + 1) ^ (c & 7)) * 16);
+  int buf = 0;    // the step's buffer
+  int tb = 0;     // KS > 1: the unit's table
+  bool ovf = false;
+  for (int i_unit = 0; U.ntiles > 0; ++i_unit) {
+    for (int g0 = 0; g0 < U.NG; g0 += kTurn) {
+      const bool last = g0 + kTurn >= U.NG;
+      const MmSrc T = last ? src_of(V) : S;      // the next turn's loads
+      const int gt = last ? 0 : g0 + kTurn;
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        if (i % Q == 0) {
+          // a step begins (its activations have landed): refill the buffer
+          // that the step before it has left
+          const int ahead = i / Q + NBUF - 1;
+          const int nb = buf + NBUF - 1 >= NBUF ? buf - 1 : buf + NBUF - 1;
+          if (ahead < D / Q) copy_x(S, g0 + ahead * Q, nb);
+          else copy_x(T, gt + (ahead - D / Q) * Q, nb);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        for (int j = 0; j < lc.nt; ++j) {
-          const int64_t t = (int64_t)lc.tr + (int64_t)lc.tg * (lc.rho * lc.tm + j);
-          dma4(lc.W + t * lc.tile_bytes + (int64_t)kb * kBlockBytes + 4 * lane,
-               lds_off(sb + 16 * P.CT * kXRow + 256 * j));
-        }
-        mm_wait_vm_all();
-        if (lane == 0) lds_write_i32(&F.ready[slot], s);
-        for (int i = 0; i < P.nl && s + 1 + i < nsteps; ++i) lc.next(F, P.njobs, JOB);
-        slot += P.nl;
-        if (slot >= P.R) slot -= P.R;
-      }
-    }
-  } else {
-    const int w = wave;
-    const int q = lane >> 4, c = lane & 15;
-    constexpr int D = mm_depth<TMX, CTX>();
-    Acc p[TMX][CTX][4];
+        v4i x[CT][2];
+        const uint32_t xo = buf * kBuf + (i % Q) * kGrp;
+        mm_read<CT>(x, x0 + xo, x1 + xo);
+        __builtin_amdgcn_sched_barrier(0);
+        v4i acc[TM][CT];
 #pragma unroll
-    for (int a = 0; a < TMX; ++a)
-#pragma unroll
-      for (int b = 0; b < CTX; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) p[a][b][e] = 0;
-    // wr[j][d]: tile j's piece of the step s with s % D == d
-    uint4 wr[TMX][D];
-    MmCur f, cur;   // next step to put in flight; the step being computed
-    f.start(F, P.njobs, JOB);
-    cur.start(F, P.njobs, JOB);
-    auto fill = [&](uint4 (&slot)[TMX][D], const int d) {
-      const bool any = f.RHO < nrounds;
-#pragma unroll
-      for (int j = 0; j < TMX; ++j) slot[j][d] = mm_issue(f, r, G, w, lane, j, any && j < f.nt);
-      if (any) f.next(F, P.njobs, JOB);
-    };
-#pragma unroll
-    for (int d = 0; d < D; ++d) fill(wr, d);
-    int s = 0, slot = 0;   // slot = s % R
-    int rdy = -1;          // the slot's ready word, read during the step before
-    for (;;) {
-#pragma unroll
-      for (int d = 0; d < D; ++d) {
-        if (s >= nsteps) goto finished;
-        const int nt = cur.nt;
-        if (rdy != s) mm_wait_word<false>(F, &F.ready[slot], s, lane);
-        const uint8_t *sb = ring + (size_t)slot * P.slot_bytes;
-        // this group's activations for the step's tokens: lane (c, q) feeds
-        // token 16 ct + c, k = 128 w + 32 q + [0, 32)
-        v4i bx[CTX][2];
-#pragma unroll
-        for (int ct = 0; ct < CTX; ++ct) {
-          const int8_t *xr = (const int8_t *)sb + (16 * ct + c) * kXRow + w * 128 + 32 * q;
-          const int4 u0 = *(const int4 *)xr, u1 = *(const int4 *)(xr + 16);
-          bx[ct][0] = v4i{u0.x, u0.y, u0.z, u0.w};
-          bx[ct][1] = v4i{u1.x, u1.y, u1.z, u1.w};
-        }
-        // Two or more column tiles: every product of the step first, then
-        // the scales -- the MFMAs' results are read only after the last one
-        // is issued, so their latency passes under the others.  One column
-        // tile: tile by tile (measured faster there).
-        v4i acc[TMX][CTX];
-        auto products = [&](int j) {
-          const uint4 wp = wr[j][d];
+        for (int j = 0; j < TM; ++j) {
+          const u4 wp = w[j][i];
           const v4i a0 = {cvt_lo16(wp.x), cvt_hi16(wp.x), cvt_lo16(wp.y), cvt_hi16(wp.y)};
           const v4i a1 = {cvt_lo16(wp.z), cvt_hi16(wp.z), cvt_lo16(wp.w), cvt_hi16(wp.w)};
 #pragma unroll
-          for (int ct = 0; ct < CTX; ++ct) {
-            if (ct < P.CT) {
-              acc[j][ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, bx[ct][0], v4i{0, 0, 0, 0}, 0,
-                                                                 0, 0);
-              acc[j][ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, bx[ct][1], acc[j][ct], 0, 0, 0);
-            }
-          }
-        };
-        auto scales = [&](int j) {
-          // this group's scales of rows 4q .. 4q+3 (row rr's 16 bytes hold
-          // the block's 8 uint16 scales)
-          const uint8_t *scl = sb + 16 * P.CT * kXRow + 256 * j;
-          Acc m[4];
+          for (int ct = 0; ct < CT; ++ct)
+            acc[j][ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[ct][0], a0, v4i{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            m[e] = mm_scale<CTX>(*(const uint16_t *)(scl + (4 * q + e) * 16 + 2 * w));
-#pragma unroll
-          for (int ct = 0; ct < CTX; ++ct) {
-            if (ct < P.CT) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) p[j][ct][e] = mm_fma(m[e], acc[j][ct][e], p[j][ct][e]);
-            }
-          }
-        };
-        if constexpr (CTX >= 2) {
-#pragma unroll
-          for (int j = 0; j < TMX; ++j)
-            if (j < nt) products(j);
-#pragma unroll
-          for (int j = 0; j < TMX; ++j)
-            if (j < nt) scales(j);
-        } else {
-#pragma unroll
-          for (int j = 0; j < TMX; ++j) {
-            if (j < nt) {
-              products(j);
-              scales(j);
-            }
-          }
+          for (int ct = 0; ct < CT; ++ct)
+            acc[j][ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[ct][1], a1, acc[j][ct], 0, 0, 0);
         }
-        // the next slot's ready word, read now so that its latency passes
-        // under this step's remaining work
-        typedef volatile __attribute__((address_space(3))) int32_t lds_i32;
-        rdy = __builtin_amdgcn_readfirstlane(
-            *(lds_i32 *)(lds_void_t *)&F.ready[slot + 1 == P.R ? 0 : slot + 1]);
-        // refill this step's registers with the step D ahead
-        fill(wr, d);
-        // the slot is free: its reads were issued before this write, and
-        // LDS instructions of a wavefront execute in order
-        if (lane == 0) mm_lds_post(&F.done[w], s);
-        if (cur.kb == cur.nblk - 1) {
-          // end of round RHO: add this wavefront's sums into its table
-          const int tb = cur.RHO & 1;
-          Acc *tbl = tables + tb * (TMX * CTX * 4 * 64);
-          mm_wait_word<true>(F, &F.tgen[tb], cur.RHO, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(T, gt + ks * D + i, i);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int jj = 0; jj < TMX; ++jj)
+        for (int j = 0; j < TM; ++j) {
+          // opaque, so that the compiler forms 32 x 32 + 64 signed multiply-adds
+          const int32_t mv = mm_opaque((int32_t)m[j][i]);
 #pragma unroll
-            for (int ct = 0; ct < CTX; ++ct)
+          for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                if (jj < nt && ct < P.CT)
-                  mm_lds_add(&tbl[((jj * CTX + ct) * 4 + e) * 64 + lane], p[jj][ct][e]);
-                p[jj][ct][e] = 0;
-              }
-          // the count follows the adds in this wavefront's LDS order, so the
-          // store wavefront, seeing it, sees the adds: neither is waited for
-          if (lane == 0) mm_lds_add_post(&F.tcnt[tb], 1);
+            for (int e = 0; e < 4; ++e)
+              p[j][ct][e] += (int64_t)mv * (int64_t)acc[j][ct][e];
         }
-        cur.next(F, P.njobs, JOB);
-        ++s;
-        if (++slot == P.R) slot = 0;
+        __builtin_amdgcn_sched_barrier(0);
+        load_m(T, gt + ks * D + i, i);
+        __builtin_amdgcn_sched_barrier(0);
+        if (i % Q == Q - 1) {
+          // the next step's activations: issued NBUF - 1 steps ago
+          mm_wait_vm<(NBUF - 2) * (ND + 2 * TM * Q) + 2 * TM * Q>();
+          if constexpr (TS > 1) __builtin_amdgcn_s_barrier();
+          __builtin_amdgcn_sched_barrier(0);
+          buf = buf + 1 == NBUF ? 0 : buf + 1;
+        }
       }
+      S = T;
     }
-  finished:;
+    // the unit's sums: rounded, checked and stored
+    const int sh = U.sh, nrows = U.nrows;
+    const int64_t half = sh > 0 ? (int64_t)1 << (sh - 1) : 0;
+    int32_t *const y32 = U.y32;
+    auto put = [&](int64_t t, int row, int tok) {
+      const int64_t v = t >> 4;   // t is 16 * the row's sum exactly
+      const int64_t a = ((v < 0 ? -v : v) + half) >> sh;
+      const int64_t y = v < 0 ? -a : a;
+      if (row < nrows && tok < B) {
+        ovf = ovf || y > 2147483647LL || y < -2147483647LL;
+        y32[(int64_t)tok * nrows + row] = (int32_t)y;
+      }
+    };
+    if constexpr (KS == 1) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int j = 0; j < TM; ++j) {
+            put(p[j][ct][e], U.row0 + (ts * TM + j) * kTileRows + c, 16 * ct + 4 * q + e);
+            p[j][ct][e] = 0;
+          }
+    } else {
+      // the slices meet in one of two LDS tables (alternating by unit, so
+      // that one barrier per unit keeps its readers and the next unit's
+      // adders apart); each wavefront stores, and clears, its share
+      int64_t *const tab = red + tb * NR;
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            mm_lds_add(tab + ((j * CT + ct) * 4 + e) * 64 + lane, p[j][ct][e]);
+            p[j][ct][e] = 0;
+          }
+      wait_lds();
+      __builtin_amdgcn_s_barrier();
+      static_assert(NR % (NW * 64) == 0, "");
+#pragma unroll
+      for (int k = 0; k < NR / (NW * 64); ++k) {
+        const int n = k * NW + wave;            // (j, ct, e)
+        int64_t *const s = tab + n * 64 + lane;
+        const int64_t t = mm_lds_take(s);
+        const int j = n / (CT * 4), ct = n / 4 % CT, e = n % 4;
+        put(t, U.row0 + j * kTileRows + c, 16 * ct + 4 * q + e);
+      }
+      tb ^= 1;
+    }
+    U = V;
+    V = unit_at(i_unit + 2);
   }
-  __syncthreads();
-  if (tid == 0) {
-    const int32_t e = lds_read_i32(&F.err);
-    if (e) atomicOr(P.err, e);
-  }
+  // copies issued past the last unit (empty ranges) have landed before the
+  // LDS is given back
+  mm_wait_vm<0>();
+  if (ovf) atomicOr(P.err, 1);
 }
 
-// The rows of a split job: y32[tok][row] = rshift_round(sum over the ns
-// slices of part / 16, sh), checked as the direct path checks it.
-struct MmFinish {
-  const int64_t *part;   // [ns][B][nrows]
-  int32_t *y32;          // [B][nrows]
-  int64_t n;             // B * nrows
-  int32_t ns, sh;
+// How a launch of `tiles` row tiles in all, the longest of NG groups, runs
+// for B tokens on ncu CUs.
+struct MmShape {
+  int CT, TM, KS, units, wgs;
 };
 
-__global__ __launch_bounds__(256) void matmul_finish_kernel(const MmFinish *fin, int32_t *err) {
-  const MmFinish &F = fin[blockIdx.y];
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= F.n) return;
-  int64_t tt = 0;
-  for (int k = 0; k < F.ns; ++k) tt += __builtin_nontemporal_load(F.part + k * F.n + i);
-  const int64_t half = F.sh > 0 ? (int64_t)1 << (F.sh - 1) : 0;
-  const int64_t v = tt >> 4;
-  const int64_t m = ((v < 0 ? -v : v) + half) >> F.sh;
-  const int64_t y = v < 0 ? -m : m;
-  if (y > 2147483647LL || y < -2147483647LL) atomicOr(err, 1);
-  F.y32[i] = (int32_t)y;
+static MmShape mm_shape(int64_t tiles, int NG, int32_t B, int ncu) {
+  MmShape s{};
+  s.CT = (B + 15) / 16;
+  // Shared where its units (4 tiles a workgroup) still fill the CUs: 768
+  // tiles (3 per CU) at B = 8, 10.0 us shared, 9.8 split; 512 tiles, 9.7 and
+  // 7.5; 1536 tiles, 14.0 and 14.4.  Beyond 32 tokens the shared copies are
+  // worth more (512 tiles, B = 48: 13.1 and 15.4; 384 tiles, K 8192: 21.0 and
+  // 21.5), and up to K = 2048 the split leaves wavefronts without groups (625
+  // tiles, K 1024, B = 24: 6.5 and 8.5).
+  const int64_t need = B > 32 || NG <= 16 ? ncu * 3 / 2 : ncu * 3;
+  s.KS = tiles >= need ? 1 : kMWaves;
+  // two tiles a wavefront share its reads of the activations, once that
+  // leaves a workgroup for every other CU: 1250 tiles, K 12288: B = 8 35.4
+  // (one tile: 34.7), B = 16 31.9 (35.6), B = 64 47.2 (54.4); 768 tiles, B =
+  // 8: 12.4 (10.0)
+  s.TM = s.KS == 1 && tiles >= (int64_t)ncu * 4 ? 2 : 1;
+  return s;
+}
+static int mm_tiles_per_unit(const MmShape &s) { return s.TM * (kMWaves / s.KS); }
+
+// Workgroups: all units at once up to two workgroups per CU.  A long pass
+// of up to 32 tokens runs one per CU: fewer streams read faster (96 FFN
+// matrices, B = 8: 463 us against 478, B = 32: 563 against 574; beyond 32
+// tokens the second workgroup's overlap is worth more: B = 64 694 against 679).
+static int mm_wgs(int units, int32_t B, int ncu) {
+  const int most = units >= 8 * ncu && B <= 32 ? ncu : 2 * ncu;
+  return units < most ? units : most;
 }
 
-// The jobs' records and the launch shape for B tokens: the grid (one
-// workgroup per CU at most), tiles per round (TMX) and column tiles of 16
-// tokens (CTX) of the kernel instance, the LDS ring and its loaders.
-static hipError_t mm_setup(const MmJobSpec *jobs, int n, int32_t B, MmJob *out,
-                           MmPlanCfg &c, bool split) {
-  if (n < 1 || B < 1 || B > 64) return hipErrorInvalidValue;
-  c.B = B;
-  c.CT = (B + 15) / 16;
-  int tmx = c.CT == 1 ? 4 : (c.CT == 2 ? 2 : 1);
+static int mm_ncu() {
   int dev = 0, ncu = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-  int maxt = 1;
+  return ncu;
+}
+
+static MmShape mm_setup(const MmJobSpec *jobs, int n, int32_t B, MmJob *out) {
+  int64_t tiles = 0;
+  int NG = 0;
+  for (int j = 0; j < n; ++j) {
+    tiles += (jobs[j].nrows + kTileRows - 1) / kTileRows;
+    NG = jobs[j].L.NG > NG ? jobs[j].L.NG : NG;
+  }
+  const int ncu = mm_ncu();
+  MmShape s = mm_shape(tiles, NG, B, ncu);
+  const int per = mm_tiles_per_unit(s);
+  int unit = 0;
   for (int j = 0; j < n; ++j) {
     MmJob &J = out[j];
     const MmJobSpec &q = jobs[j];
     J = MmJob{};
-    J.W = q.w;
-    J.x8 = q.x8;
-    J.y32 = q.y32;
-    J.tile_bytes = q.L.tile_bytes;
-    J.nrows = q.nrows;
-    J.ntiles = (q.nrows + kTileRows - 1) / kTileRows;
-    J.NG = q.L.NG;
-    J.nblk = q.L.nblk;
-    J.sh = q.sh;
-    J.K = q.L.K;
-    J.ns = 1;
-    maxt = J.ntiles > maxt ? J.ntiles : maxt;
+    J.u.W = q.w;
+    J.u.x8 = q.x8;
+    J.u.y32 = q.y32;
+    J.u.tile_bytes = (int32_t)q.L.tile_bytes;
+    J.u.nrows = q.nrows;
+    J.u.ntiles = (q.nrows + kTileRows - 1) / kTileRows;
+    J.u.NG = q.L.NG;
+    J.u.sh = q.sh;
+    J.u.K = q.L.K;
+    J.unit0 = unit;
+    unit += (J.u.ntiles + per - 1) / per;
   }
-  const int G = maxt < ncu ? maxt : ncu;
-  // A matrix with at most one tile per workgroup and enough tiles to give
-  // every workgroup one K slice of one (a 4096-row down projection on 256
-  // workgroups) is split into ns K slices when the caller has reduction
-  // buffers for it (a plan): ns = 4 for up to 16 tokens, 2 for up to 32.
-  const int ns_want = c.CT == 1 ? 4 : (c.CT == 2 ? 2 : 1);
-  std::vector<int> per(n);
-  for (int j = 0; j < n; ++j) {
-    MmJob &J = out[j];
-    per[j] = (J.ntiles + G - 1) / G;
-    if (split && ns_want > 1 && per[j] == 1 && J.nblk % ns_want == 0 && G % ns_want == 0 &&
-        J.ntiles * ns_want >= G) {
-      J.ns = ns_want;
-      per[j] = (J.ntiles + G / ns_want - 1) / (G / ns_want);
-    }
-  }
-  // one tile per workgroup in every job: rounds of one tile, with the deeper
-  // weight pipeline of the one-tile kernels; three a workgroup at 17..32
-  // tokens (as a 12288-row matrix has on 256 workgroups): rounds of three, so
-  // that one copy of a block's activations serves all three
-  int maxper = 1;
-  for (int j = 0; j < n; ++j) maxper = per[j] > maxper ? per[j] : maxper;
-  if (maxper == 1) tmx = 1;
-  else if (c.CT == 2 && maxper == 3) tmx = 3;
-  const int ctxt = tmx == 4 ? 1 : (tmx >= 2 ? c.CT : (c.CT <= 2 ? c.CT : 4));
-  const int table_bytes = 2 * tmx * ctxt * 4 * 64 * 8;
-  c.slot_bytes = 16 * c.CT * kXRow + tmx * 256;
-  const int avail = kLdsBytes - kFlagBytes - table_bytes;
-  c.R = avail / c.slot_bytes;
-  if (c.R > kRingMax) c.R = kRingMax;
-  if (c.R < 2) return hipErrorInvalidValue;
-  c.nl = c.R - 1 < kML ? c.R - 1 : kML;   // >= 1: R >= 2
-  // rounds of tm tiles: as many tiles per round as the workgroups' shares
-  // of the job allow, at most tmx
-  for (int j = 0; j < n; ++j) out[j].tm = per[j] < tmx ? per[j] : tmx;
-  c.G = G;
-  c.tmx = tmx;
-  c.ctxt = ctxt;
-  c.lds = (size_t)kFlagBytes + table_bytes + (size_t)c.R * c.slot_bytes;
-  return hipSuccess;
+  s.units = unit;
+  s.wgs = mm_wgs(unit, B, ncu);
+  return s;
 }
 
-template <bool kTab>
-static hipError_t mm_set_lds_limit() {
-  hipError_t e = hipFuncSetAttribute((const void *)matmul_kernel<4, 1, kTab>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *)matmul_kernel<2, 2, kTab>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *)matmul_kernel<3, 2, kTab>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *)matmul_kernel<1, 4, kTab>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *)matmul_kernel<1, 1, kTab>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute((const void *)matmul_kernel<1, 2, kTab>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
-  return e;
-}
-
-template <bool kTab>
-static hipError_t mm_launch(const MmParams &P, const MmPlanCfg &c, hipStream_t s) {
+template <int TM, int CT, int KS, bool half8, bool plan>
+static hipError_t mm_launch1(const MmParams &P, int wgs, hipStream_t s) {
+  auto *const k = &matmul_kernel<TM, CT, KS, half8, plan>;
   // dynamic LDS beyond the default limit: allowed once per process
-  static const hipError_t attr = mm_set_lds_limit<kTab>();
+  static const hipError_t attr = hipFuncSetAttribute(
+      (const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
   if (attr != hipSuccess) return attr;
-  const dim3 g(c.G), b(kMThreads);
-  if (c.tmx == 4) {
-    hipLaunchKernelGGL((matmul_kernel<4, 1, kTab>), g, b, c.lds, s, P);
-  } else if (c.tmx == 3) {
-    hipLaunchKernelGGL((matmul_kernel<3, 2, kTab>), g, b, c.lds, s, P);
-  } else if (c.tmx == 2) {
-    hipLaunchKernelGGL((matmul_kernel<2, 2, kTab>), g, b, c.lds, s, P);
-  } else if (c.ctxt == 1) {
-    hipLaunchKernelGGL((matmul_kernel<1, 1, kTab>), g, b, c.lds, s, P);
-  } else if (c.ctxt == 2) {
-    hipLaunchKernelGGL((matmul_kernel<1, 2, kTab>), g, b, c.lds, s, P);
-  } else {
-    hipLaunchKernelGGL((matmul_kernel<1, 4, kTab>), g, b, c.lds, s, P);
-  }
+  constexpr size_t lds = mm_x_bytes(CT, KS, half8) +
+                         (KS > 1 ? (size_t)2 * TM * CT * 4 * 64 * sizeof(int64_t) : 0);
+  static_assert(lds <= kLdsBytes, "LDS of one workgroup");
+  hipLaunchKernelGGL(k, dim3(wgs), dim3(kMThreads), lds, s, P);
   return hipGetLastError();
 }
 
-static void mm_params(MmParams &P, int n, const MmPlanCfg &c, int32_t *err) {
-  P.njobs = n;
-  P.B = c.B;
-  P.CT = c.CT;
-  P.R = c.R;
-  P.nl = c.nl;
-  P.slot_bytes = c.slot_bytes;
-  P.err = err;
+template <int CT, bool plan>
+static hipError_t mm_launch2(const MmParams &P, const MmShape &c, hipStream_t s) {
+  if constexpr (CT == 1) {
+    // the split's private copies are halved for up to 8 tokens
+    if (c.KS > 1 && P.B <= 8) return mm_launch1<1, CT, kMWaves, true, plan>(P, c.wgs, s);
+  }
+  if (c.KS > 1) return mm_launch1<1, CT, kMWaves, false, plan>(P, c.wgs, s);
+  return c.TM == 1 ? mm_launch1<1, CT, 1, false, plan>(P, c.wgs, s)
+                   : mm_launch1<2, CT, 1, false, plan>(P, c.wgs, s);
+}
+
+template <bool plan>
+static hipError_t mm_launch(const MmParams &P, const MmShape &c, hipStream_t s) {
+  switch (c.CT) {
+    case 1: return mm_launch2<1, plan>(P, c, s);
+    case 2: return mm_launch2<2, plan>(P, c, s);
+    case 3: return mm_launch2<3, plan>(P, c, s);
+    case 4: return mm_launch2<4, plan>(P, c, s);
+    default: return hipErrorInvalidValue;   // 1..64 tokens
+  }
 }
 
 }  // namespace
 
-size_t matmul_job_bytes() { return sizeof(MmJob); }
-
-hipError_t matmul_plan_prepare(const MmJobSpec *jobs, int n, int32_t B, void *table,
-                               MmPlanCfg *cfg, int32_t *ns) {
-  if (n < 1 || n > kMmPlanJobs || !table || !cfg || !ns) return hipErrorInvalidValue;
-  const hipError_t e = mm_setup(jobs, n, B, (MmJob *)table, *cfg, true);
-  for (int j = 0; e == hipSuccess && j < n; ++j) ns[j] = ((const MmJob *)table)[j].ns;
-  return e;
+hipError_t matmul_plan_prepare(const MmJobSpec *jobs, int n, int32_t B,
+                               std::vector<uint8_t> &table, MmPlanCfg *cfg) {
+  if (n < 1 || n > kMmPlanJobs || B < 1 || B > 64 || !cfg) return hipErrorInvalidValue;
+  std::vector<MmJob> J(n);
+  const MmShape s = mm_setup(jobs, n, B, J.data());
+  const int per = mm_tiles_per_unit(s);
+  // The units one after another, those of the longest matrices first:
+  // workgroup r takes units r, r + wgs, ..., so the shares differ by less
+  // than one unit of each K.
+  std::vector<int> order(n);
+  for (int j = 0; j < n; ++j) order[j] = j;
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int a, int b) { return J[a].u.NG > J[b].u.NG; });
+  table.resize((size_t)s.units * sizeof(MmUnit));
+  MmUnit *out = (MmUnit *)table.data();
+  for (int j : order)
+    for (int t = 0; t < J[j].u.ntiles; t += per) {
+      MmUnit &u = *out++;
+      u = J[j].u;
+      u.W += (int64_t)t * u.tile_bytes;
+      u.ntiles -= t;
+      u.row0 = t * kTileRows;
+    }
+  *cfg = MmPlanCfg{B, s.CT, s.TM, s.KS, s.units, s.wgs};
+  return hipSuccess;
 }
 
-void matmul_plan_bind(void *table, int j, int64_t *part) { ((MmJob *)table)[j].part = part; }
-
-size_t matmul_finish_bytes() { return sizeof(MmFinish); }
-
-int matmul_finish_prepare(const void *table, int n, int32_t B, void *fin) {
-  int nf = 0;
-  for (int j = 0; j < n; ++j) {
-    const MmJob &J = ((const MmJob *)table)[j];
-    if (J.ns <= 1) continue;
-    MmFinish &f = ((MmFinish *)fin)[nf++];
-    f.part = J.part;
-    f.y32 = J.y32;
-    f.n = (int64_t)B * J.nrows;
-    f.ns = J.ns;
-    f.sh = J.sh;
-  }
-  return nf;
-}
-
-hipError_t launch_matmul_finish(const void *d_fin, int nf, int64_t max_n, int32_t *err,
-                                hipStream_t s) {
-  if (nf < 1) return hipSuccess;
-  const dim3 g((unsigned)((max_n + 255) / 256), (unsigned)nf);
-  hipLaunchKernelGGL(matmul_finish_kernel, g, dim3(256), 0, s, (const MmFinish *)d_fin, err);
-  return hipGetLastError();
-}
-
-hipError_t launch_matmul_plan(const void *d_table, int n, const MmPlanCfg &cfg, int32_t *err,
+hipError_t launch_matmul_plan(const void *d_table, const MmPlanCfg &cfg, int32_t *err,
                               hipStream_t s) {
-  if (n < 1 || n > kMmPlanJobs || !d_table) return hipErrorInvalidValue;
+  if (!d_table) return hipErrorInvalidValue;
   MmParams P{};
-  mm_params(P, n, cfg, err);
-  P.tab = (const MmJob *)d_table;
-  return mm_launch<true>(P, cfg, s);
+  P.units = cfg.units;
+  P.B = cfg.B;
+  P.err = err;
+  P.tab = (const MmUnit *)d_table;
+  return mm_launch<true>(P, MmShape{cfg.CT, cfg.TM, cfg.KS, cfg.units, cfg.wgs}, s);
 }
 
 hipError_t launch_matmul_multi(const MmJobSpec *jobs, int n, int32_t B, int32_t *err,
                                hipStream_t s) {
-  if (n < 1 || n > kMmJobs) return hipErrorInvalidValue;
+  if (n < 1 || n > kMmJobs || B < 1 || B > 64) return hipErrorInvalidValue;
   MmParams P{};
-  MmPlanCfg c{};
-  hipError_t e = mm_setup(jobs, n, B, P.job, c, false);
-  if (e != hipSuccess) return e;
-  mm_params(P, n, c, err);
+  const MmShape c = mm_setup(jobs, n, B, P.job);
+  P.njobs = n;
+  P.units = c.units;
+  P.B = B;
+  P.err = err;
   return mm_launch<false>(P, c, s);
 }
 
