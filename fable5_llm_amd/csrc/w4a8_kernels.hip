@@ -18,240 +18,363 @@ namespace w4a8 {
 // threads take pieces of 8 elements: thread t holds elements
 // [c*NT*8 + 8t, +8) of piece c, so the 4 threads of a DPP quad hold 32
 // consecutive elements -- one (group, k-quarter) of the weight layout.
+//
+// It stands between a launch's start and its first dot product, one chain of
+// load, reductions and arithmetic on a few wavefronts, so its length is its
+// instruction count and its LDS round trips.  One kernel instance per
+// prologue kind, no branch per element: 16-bit steps run two elements an
+// instruction (v_pk_*_i16), wide products are 32 x 32 + 64 multiply-adds on
+// magnitudes, and a reduction is one LDS round trip (GroupRed).  From the
+// first workgroup's start to the first dot product, K = 4096: DYNQ8 3.3 ->
+// 2.4 us, RMSNorm 5.6 -> 3.9 us; a layer's FFN block 25.3 -> 23.4 us, the
+// chained step in graph mode 1.405 -> 1.306 ms.
 // ---------------------------------------------------------------------------
-// v has been loaded: uses after this point need no wait, and no memory
-// access is moved above it
-__device__ __forceinline__ void arrived(int4 &v) {
-  int a = v.x, b = v.y, c = v.z, d = v.w;
-  asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d) :: "memory");
-  v = make_int4(a, b, c, d);
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ s16x2 as_s16x2(int v) { return __builtin_bit_cast(s16x2, v); }
+__device__ __forceinline__ int piece_word(const int4 &p, int i) {
+  return i == 0 ? p.x : (i == 1 ? p.y : (i == 2 ? p.z : p.w));
+}
+__device__ __forceinline__ int pack16(int lo, int hi) {
+  return (int)__builtin_amdgcn_perm((uint32_t)hi, (uint32_t)lo, 0x05040100u);
 }
 
-template <int NT>
+// clip16 of a magnitude with its sign
+__device__ __forceinline__ int32_t clip16_mag(uint32_t q, bool neg) {
+  const int32_t m = (int32_t)min(q, 32767u + (neg ? 1u : 0u));
+  return neg ? -m : m;
+}
+
+// ALU EMUL32 at p0 = 12 (gen_layer_script.py:1414-1418):
+// clip16(rshift_round(a * b, 12)), b int16
+__device__ __forceinline__ int32_t emul12(int32_t a, int32_t b) {
+  static_assert(kEmulP0 == 12, "");
+  const uint32_t ma = a < 0 ? 0u - (uint32_t)a : (uint32_t)a, mb = (uint32_t)abs(b);
+  const uint64_t v = (uint64_t)ma * mb + 2048u;     // |a * b| <= 2^46
+  const uint32_t q = (uint32_t)(v >> 32) ? 0xFFFFFFFFu : (uint32_t)v;
+  return clip16_mag(q >> 12, (a ^ b) < 0);
+}
+
+// 1/sqrt(v * 2^-P) ~= r * 2^(e-30), v >= 1: fixedpoint.py:56-75.  Every value
+// of its int64 steps fits 32 bits (m < 2^32, r and r^2 >> 30 at most 2^30,
+// m r^2 near 2^30), so each step is one 32 x 32 -> 64 product.
+template <typename T>
+__device__ __forceinline__ void rsqrt32(uint64_t v, int P, const T *lut, uint32_t *r_out,
+                                        int *e_out) {
+  int s = 32 - __clzll((long long)v);
+  if ((s - P) & 1) s += 1;
+  const uint32_t m = (uint32_t)(s >= 0 ? (v >> s) : (v << (-s)));
+  const uint32_t idx = m < 0x80000000u ? (m >> 22) & 0xFFu : 256u | ((m >> 23) & 0xFFu);
+  uint32_t r = (uint32_t)lut[idx] << 15;
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const uint32_t r2 = (uint32_t)(((uint64_t)r * r) >> 30);
+    const uint32_t mr2 = (uint32_t)(((uint64_t)m * r2) >> 30);
+    r = (uint32_t)(((uint64_t)r * (0xC0000000u - mr2)) >> 31);
+  }
+  *r_out = r;
+  *e_out = -((s - P + 30) / 2);
+}
+
+template <int PRO, int NT>
 struct ProRegs {
-  static constexpr int kPc = (kKMax + NT * 8 - 1) / (NT * 8);   // int16 pieces
-  static constexpr int kNw = (8192 + NT * 8 - 1) / (NT * 8);    // norm pieces (K <= 8192)
-  int4 pc[kPc];   // int16 x (PRO_X8: 16 int8 per piece)
-  int4 wv[kNw];   // int16 RMSNorm weights
+  static constexpr int kPer = PRO == PRO_X8 ? 16 : 8;            // elements of a piece
+  static constexpr int kK = PRO == PRO_RMSNORM_DYNQ8 ? 8192 : kKMax;
+  static constexpr int kPc = (kK + NT * kPer - 1) / (NT * kPer);
+  int4 pc[kPc];   // int16 x (PRO_X8: 16 int8 per piece), zeros past K
+  int4 wv[PRO == PRO_RMSNORM_DYNQ8 ? kPc : 1];   // int16 RMSNorm weights
 };
 
-// The activation loads are issued before any weight load, so they are not
-// queued behind the weight stream.  Every piece is loaded without a branch
-// (the address clamped to the vector), so all of a thread's loads are in
-// flight together and one wait covers them; pieces past K are zeroed by
-// pro_mask, at first use, so nothing between the two waits for the loads.
-template <int NT>
-__device__ __forceinline__ void pro_load(const GemvParams &P, ProRegs<NT> &X, int tid) {
-  const int K = P.K;
-  if (P.pro == PRO_X8) {
-    const int8_t *x = (const int8_t *)P.x;
-#pragma unroll
-    for (int c = 0; c < ProRegs<NT>::kPc; ++c) {
-      const int i = (c * NT + tid) * 16;
-      X.pc[c] = *(const int4 *)(x + (i < K ? i : K - 16));
-    }
-    return;
-  }
-  const int16_t *x16 = (const int16_t *)P.x;
-#pragma unroll
-  for (int c = 0; c < ProRegs<NT>::kPc; ++c) {
-    const int base = c * NT * 8 + tid * 8;
-    X.pc[c] = *(const int4 *)(x16 + (base < K ? base : K - 8));
-  }
-  if (P.pro == PRO_EMUL_DYNQ8) {
-    // the product is formed here, so the prologue group waits for its
-    // loads now; the weight wavefronts already have their blocks in flight
-    int4 a[ProRegs<NT>::kPc][2];
-#pragma unroll
-    for (int c = 0; c < ProRegs<NT>::kPc; ++c) {
-      const int base = c * NT * 8 + tid * 8;
-      const int32_t *p = P.x2 + (base < K ? base : K - 8);
-      a[c][0] = *(const int4 *)p;
-      a[c][1] = *(const int4 *)(p + 4);
-    }
-#pragma unroll
-    for (int c = 0; c < ProRegs<NT>::kPc; ++c) {
-      const int32_t av[8] = {a[c][0].x, a[c][0].y, a[c][0].z, a[c][0].w,
-                             a[c][1].x, a[c][1].y, a[c][1].z, a[c][1].w};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int64_t v = movy_shift((int64_t)av[j] * piece_get(X.pc[c], j), kEmulP0);
-        piece_set(X.pc[c], j, (int16_t)clamp64(v, -32768, 32767));
-      }
-    }
-  }
-  if (P.pro == PRO_RMSNORM_DYNQ8) {
-#pragma unroll
-    for (int c = 0; c < ProRegs<NT>::kNw; ++c) {
-      const int base = c * NT * 8 + tid * 8;
-      X.wv[c] = *(const int4 *)(P.norm_w + (base < K ? base : K - 8));
-    }
-  }
-}
-
-template <int NT>
-__device__ __forceinline__ void pro_mask(const GemvParams &P, ProRegs<NT> &X, int tid) {
+// the loads of x (and of the norm weights): issued before any weight load
+template <int PRO, int NT>
+__device__ __forceinline__ void pro_load(const GemvParams &P, ProRegs<PRO, NT> &X, int tid) {
+  typedef ProRegs<PRO, NT> R;
   const int K = P.K;
   const int4 z = make_int4(0, 0, 0, 0);
-  const int per = P.pro == PRO_X8 ? 16 : 8;
 #pragma unroll
-  for (int c = 0; c < ProRegs<NT>::kPc; ++c)
-    if ((c * NT + tid) * per >= K) X.pc[c] = z;
-  if (P.pro == PRO_RMSNORM_DYNQ8)
+  for (int c = 0; c < R::kPc; ++c) {
+    const int i = (c * NT + tid) * R::kPer;
+    X.pc[c] = z;
+    if constexpr (PRO == PRO_RMSNORM_DYNQ8) X.wv[c] = z;
+    if (i < K) {
+      if constexpr (PRO == PRO_X8) X.pc[c] = *(const int4 *)((const int8_t *)P.x + i);
+      else X.pc[c] = *(const int4 *)((const int16_t *)P.x + i);
+      if constexpr (PRO == PRO_RMSNORM_DYNQ8) X.wv[c] = *(const int4 *)(P.norm_w + i);
+    }
+  }
+  if constexpr (PRO == PRO_EMUL_DYNQ8) {
+    int4 a[R::kPc][2];
 #pragma unroll
-    for (int c = 0; c < ProRegs<NT>::kNw; ++c)
-      if ((c * NT + tid) * 8 >= K) X.wv[c] = z;
+    for (int c = 0; c < R::kPc; ++c) {
+      const int i = (c * NT + tid) * 8;
+      a[c][0] = a[c][1] = z;
+      if (i < K) {
+        a[c][0] = *(const int4 *)(P.x2 + i);
+        a[c][1] = *(const int4 *)(P.x2 + i + 4);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < R::kPc; ++c)
+      if (c * NT * 8 < K) {
+        const int av[8] = {a[c][0].x, a[c][0].y, a[c][0].z, a[c][0].w,
+                           a[c][1].x, a[c][1].y, a[c][1].z, a[c][1].w};
+        int o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const s16x2 g = as_s16x2(piece_word(X.pc[c], i));
+          o[i] = pack16(emul12(av[2 * i], g.x), emul12(av[2 * i + 1], g.y));
+        }
+        X.pc[c] = make_int4(o[0], o[1], o[2], o[3]);
+      }
+  }
 }
 
-// The prologue's barrier when the whole workgroup runs it.
-struct WgSync {
-  __device__ void operator()() const { __syncthreads(); }
+// The prologue's reductions over its wavefronts when the whole workgroup
+// runs it (sm: 2 * NW int64 of LDS).
+template <int NW>
+struct WgRed {
+  int64_t *sm;
+  __device__ uint64_t sum(uint64_t v, int wave, int lane) {
+    if (lane == 0) sm[wave] = (int64_t)v;
+    __syncthreads();
+    uint64_t t = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) t += (uint64_t)sm[w];
+    return t;
+  }
+  __device__ int32_t max(int32_t v, int wave, int lane) {
+    if (lane == 0) sm[NW + wave] = v;
+    __syncthreads();
+    int32_t t = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) t = ::max(t, (int32_t)sm[NW + w]);
+    return t;
+  }
+  __device__ void done(int, int) { __syncthreads(); }
 };
 
-// sm: 2 * NT / 64 int64 of LDS.  Leaves x8 in xs[0, K) and the offset
-// corrections -8 * (sum of the x8 met by the offset-form low nibbles of
-// each (group, k-quarter)) in xlo; returns e_x.  sync() is a barrier of the
-// NT threads.
-template <int NT, typename TabT, typename Sync>
-__device__ int pro_compute(const GemvParams &P, ProRegs<NT> &X, int8_t *xs, int32_t *xlo,
-                           int64_t *sm, const TabT *rsqrt_lut, int tid, Sync &sync) {
-  constexpr int NW = NT / 64;
+// ... and when 8 wavefronts of a larger workgroup run it: no workgroup
+// barrier, since the others may be stalled behind their weight loads.  Each
+// wavefront posts its value with a valid bit, and polls the eight words until
+// all have it: one LDS round trip for value and flag, the eight lanes of a
+// half row holding the eight values.
+struct ProWords {
+  uint64_t sum[8];    // zero at the launch's start; bit 63: valid
+  uint32_t max[8];    // bit 31: valid
+  int32_t ready[8];   // the wavefront's share of x8 is stored
+};
+__device__ __forceinline__ uint64_t lds_read_u64(const uint64_t *p) {
+  uint64_t v;
+  asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(lds_off(p)) : "memory");
+  return v;
+}
+__device__ __forceinline__ void lds_post_u64(uint64_t *p, uint64_t v) {
+  asm volatile("ds_write_b64 %0, %1" :: "v"(lds_off(p)), "v"(v) : "memory");
+}
+__device__ __forceinline__ void lds_post_i32(int32_t *p, int32_t v) {
+  asm volatile("ds_write_b32 %0, %1" :: "v"(lds_off(p)), "v"(v) : "memory");
+}
+struct GroupRed {
+  ProWords *w;
+  bool ok;    // false once a poll gave up
+  __device__ uint64_t sum(uint64_t v, int wave, int lane) {
+    if (lane == 0) lds_post_u64(&w->sum[wave], v | (1ull << 63));
+    uint64_t t = 0;
+    bool got = false;
+    for (uint32_t n = 0; n < kLdsSpin && !got; ++n) {
+      t = lds_read_u64(&w->sum[lane & 7]);
+      got = __all((int64_t)t < 0);
+    }
+    ok = ok && got;
+    t &= ~(1ull << 63);
+    t += dpp_u64<0xB1, 0xF>(t);    // pairs, quads, half rows
+    t += dpp_u64<0x4E, 0xF>(t);
+    t += dpp_u64<0x141, 0xF>(t);
+    return t;
+  }
+  __device__ int32_t all_max(int lane) {
+    int32_t t = 0;
+    bool got = false;
+    for (uint32_t n = 0; n < kLdsSpin && !got; ++n) {
+      t = lds_read_i32((const int32_t *)&w->max[lane & 7]);
+      got = __all(t < 0);
+    }
+    ok = ok && got;
+    t &= 0x7FFFFFFF;
+    t = ::max(t, W4A8_DPP(t, 0, 0xB1, 0xF));
+    t = ::max(t, W4A8_DPP(t, 0, 0x4E, 0xF));
+    return ::max(t, W4A8_DPP(t, 0, 0x141, 0xF));
+  }
+  __device__ int32_t max(int32_t v, int wave, int lane) {
+    if (lane == 0) lds_post_i32((int32_t *)&w->max[wave], v | (int32_t)0x80000000);
+    return all_max(lane);
+  }
+  // every wavefront's share of x8 is stored (a wavefront's LDS instructions
+  // execute in order); backoff: 64 cycles between polls
+  template <bool backoff = false>
+  __device__ void wait_ready(int lane) {
+    bool got = false;
+    for (uint32_t n = 0; n < kLdsSpin && !got; ++n) {
+      got = __all(lds_read_i32(&w->ready[lane & 7]) != 0);
+      if (backoff && !got) __builtin_amdgcn_s_sleep(1);
+    }
+    ok = ok && got;
+  }
+  __device__ void done(int wave, int lane) {
+    if (lane == 0) lds_post_i32(&w->ready[wave], 1);
+    wait_ready(lane);
+  }
+};
+
+// A workgroup barrier that waits for LDS alone: __syncthreads may also wait
+// for the weight loads in flight.
+__device__ __forceinline__ void meet() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// fixedpoint.py:24-33: the least e with rshift_round(max, e) <= 127 is
+// bitlen(max) - 7, or one more when rounding carries past 127
+__device__ __forceinline__ int dynq8_exponent(int32_t mx) {
+  int e = mx > 127 ? 25 - __clz(mx) : 0;
+  if (e > 0 && ((mx + (1 << (e - 1))) >> e) > 127) ++e;
+  return e;
+}
+
+// Leaves x8 in xs[0, K) and the offset corrections -8 * (sum of the x8 met by
+// the offset-form low nibbles of each (group, k-quarter)) in xlo; returns e_x.
+template <int PRO, int NT, typename TabT, typename Red>
+__device__ __forceinline__ int pro_compute(const GemvParams &P, ProRegs<PRO, NT> &X, int8_t *xs,
+                                           int32_t *xlo, const TabT *rsqrt_lut, int tid,
+                                           Red &red) {
+  typedef ProRegs<PRO, NT> R;
   const int K = P.K;
   const int lane = tid & 63, wave = tid >> 6;
   const bool writer = blockIdx.x == 0;
-  pro_mask<NT>(P, X, tid);
-  if (P.pro == PRO_X8) {
-    const int np = (K + NT * 16 - 1) / (NT * 16);
+  if constexpr (PRO == PRO_X8) {
 #pragma unroll
-    for (int c = 0; c < ProRegs<NT>::kPc; ++c) {
+    for (int c = 0; c < R::kPc; ++c) {
       const int i = (c * NT + tid) * 16;
-      if (c < np && i < K) {
+      // the two threads of a pair hold one (group, k-quarter)
+      int s = __builtin_amdgcn_sdot4(X.pc[c].x, 0x01010101, 0, false);
+      s = __builtin_amdgcn_sdot4(X.pc[c].z, 0x01010101, s, false);
+      s += W4A8_DPP(s, 0, 0xB1, 0xF);
+      if (i < K) {
         *(int4 *)(xs + i) = X.pc[c];
+        if ((tid & 1) == 0) xlo[i / 32] = -8 * s;
         if (writer && P.x8_out) *(int4 *)(P.x8_out + i) = X.pc[c];
       }
     }
-    sync();
-    for (int c = tid; c < P.NG * 4; c += NT) {
-      const int *xw = (const int *)(xs + 32 * c);
-      int s = 0;
-      s = __builtin_amdgcn_sdot4(xw[0], 0x01010101, s, false);
-      s = __builtin_amdgcn_sdot4(xw[2], 0x01010101, s, false);
-      s = __builtin_amdgcn_sdot4(xw[4], 0x01010101, s, false);
-      s = __builtin_amdgcn_sdot4(xw[6], 0x01010101, s, false);
-      xlo[c] = -8 * s;
-    }
     if (writer && P.e_x_out && tid == 0) *P.e_x_out = P.e_x_given;
-    sync();
+    red.done(wave, lane);
     return P.e_x_given;
   }
-  const int np = (K + NT * 8 - 1) / (NT * 8);
-  if (P.pro == PRO_RMSNORM_DYNQ8) {
+  if constexpr (PRO == PRO_RMSNORM_DYNQ8) {
     // layer_fixed.py:1262-1278 in sign-magnitude form: rshift_round rounds
     // the magnitude, so |x * r| and |y * sc| carry the rounding and the
     // sign is restored afterwards
     uint64_t ss = 0;
 #pragma unroll
-    for (int c = 0; c < ProRegs<NT>::kNw; ++c)
-      if (c < np)
+    for (int c = 0; c < R::kPc; ++c)
 #pragma unroll
-        for (int j = 0; j < 8; j += 2) {
-          const int32_t a = piece_get(X.pc[c], j), b = piece_get(X.pc[c], j + 1);
-          ss += (uint64_t)((uint32_t)(a * a) + (uint32_t)(b * b));
-        }
-    ss = wave_sum_u64(ss);
-    if (lane == 0) sm[wave] = (int64_t)ss;
-    sync();
-    ss = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) ss += (uint64_t)sm[w];
+      for (int i = 0; i < 4; ++i) {
+        const s16x2 v = as_s16x2(piece_word(X.pc[c], i));
+        ss += (uint32_t)__builtin_amdgcn_sdot2(v, v, 0, false);   // at most 2^31
+      }
+    ss = red.sum(wave_sum_u64(ss), wave, lane);
     if (ss == 0) ss = 1;
-    int64_t r;
+    uint32_t r;
     int e;
-    rsqrt_q(ss, 2 * P.in_f + (31 - __clz(K)), rsqrt_lut, &r, &e);
+    rsqrt32(ss, 2 * P.in_f + (31 - __clz(K)), rsqrt_lut, &r, &e);
+    // r < 2^31 (a Q30 reciprocal square root) and |x| <= 2^15; for in_f in
+    // 0..40 (checked on the host) a left shift is at most 17, so the shifted
+    // |x| * r stays below 2^63
     const int s1 = 30 - e;
     const int32_t one = P.one_plus ? (1 << 14) : 0;
-    const int rs = s1 < 0 ? 0 : (s1 > 63 ? 63 : s1);
-    const int ls = s1 < 0 ? (-s1 > 63 ? 63 : -s1) : 0;
+    const int rs = s1 < 0 ? 0 : (s1 > 63 ? 63 : s1), ls = s1 < 0 ? -s1 : 0;
     const uint64_t half1 = rs > 0 ? ((uint64_t)1 << (rs - 1)) : 0;
-    const bool right = s1 >= 0;
-    // r < 2^31 (a Q30 reciprocal square root) and |x| <= 2^15; for in_f in
-    // 0..40 (checked on the host) the left shift is at most 17, so the
-    // shifted |x| * r stays below 2^63
-    const uint32_t r32 = (uint32_t)r;
+    auto norm = [&](int32_t xv, int32_t wv, bool left) {
+      const int32_t sc = wv + one;
+      const uint64_t mag = (uint64_t)(uint32_t)abs(xv) * (uint64_t)r + half1;
+      const uint64_t ym = left ? mag << ls : mag >> rs;
+      // y is clipped to [-2^32, 2^32 - 1]; a magnitude of 2^32 or more
+      // saturates the int16 result for any nonzero scale exactly as
+      // 2^32 - 1 does, so the product is formed in 32 x 32 bits
+      const uint32_t y = (uint32_t)(ym >> 32) ? 0xFFFFFFFFu : (uint32_t)ym;
+      const uint64_t qv = (uint64_t)y * (uint64_t)(uint32_t)abs(sc) + 8192u;
+      // qv >> 14, saturated: above 2^32 it is past the clip
+      const uint32_t q = (uint32_t)(qv >> 32) ? 0xFFFFFFFFu : (uint32_t)qv;
+      return clip16_mag(q >> 14, (xv ^ sc) < 0);
+    };
+    auto pieces = [&](bool left) {
 #pragma unroll
-    for (int c = 0; c < ProRegs<NT>::kNw; ++c) {
-      const int base = c * NT * 8 + tid * 8;
-      if (c < np) {
+      for (int c = 0; c < R::kPc; ++c)
+        if (c * NT * 8 < K) {
+          int o[4];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int32_t xv = piece_get(X.pc[c], j);
-          const int32_t sc = (int32_t)piece_get(X.wv[c], j) + one;
-          const uint64_t mag = (uint64_t)(uint32_t)abs(xv) * (uint64_t)r32;
-          uint64_t ym = right ? ((mag + half1) >> rs) : (mag << ls);
-          // y is clipped to [-2^32, 2^32 - 1]; a magnitude of 2^32 or more
-          // saturates the int16 result for any nonzero scale exactly as
-          // 2^32 - 1 does, so the product is formed in 32 x 32 bits
-          ym = ym < 0xFFFFFFFFull ? ym : 0xFFFFFFFFull;
-          const uint64_t qv = ((uint64_t)(uint32_t)ym * (uint64_t)(uint32_t)abs(sc) + 8192u) >> 14;
-          const bool neg = (xv < 0) != (sc < 0);
-          const int32_t q32 = qv > 65535u ? 65535 : (int32_t)qv;
-          const int32_t qm = min(q32, 32767 + (int32_t)neg);
-          piece_set(X.pc[c], j, (int16_t)(neg ? -qm : qm));
+          for (int i = 0; i < 4; ++i) {
+            const s16x2 v = as_s16x2(piece_word(X.pc[c], i)), w = as_s16x2(piece_word(X.wv[c], i));
+            o[i] = pack16(norm(v.x, w.x, left), norm(v.y, w.y, left));
+          }
+          X.pc[c] = make_int4(o[0], o[1], o[2], o[3]);
+          const int base = (c * NT + tid) * 8;
+          if (writer && P.xn_out && base < K) *(int4 *)(P.xn_out + base) = X.pc[c];
         }
-        if (writer && P.xn_out && base < K) *(int4 *)(P.xn_out + base) = X.pc[c];
-      }
-    }
+    };
+    if (s1 >= 0) pieces(false);
+    else pieces(true);
   }
-  int32_t mx = 0;
+  s16x2 hi = {0, 0}, lo = {0, 0};
 #pragma unroll
-  for (int c = 0; c < ProRegs<NT>::kPc; ++c)
-    if (c < np)
+  for (int c = 0; c < R::kPc; ++c)
+    if (c * NT * 8 < K)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) mx = max(mx, abs((int32_t)piece_get(X.pc[c], j)));
-  mx = wave_max_i32(mx);
-  if (lane == 0) sm[NW + wave] = mx;
-  sync();
-  mx = 0;
-#pragma unroll
-  for (int w = 0; w < NW; ++w) mx = max(mx, (int32_t)sm[NW + w]);
-  // fixedpoint.py:24-33: the least e with rshift_round(max, e) <= 127 is
-  // bitlen(max) - 7, or one more when rounding carries past 127
-  int e = mx > 127 ? 25 - __clz(mx) : 0;
-  if (e > 0 && ((mx + (1 << (e - 1))) >> e) > 127) ++e;
-  const int32_t half = (1 << e) >> 1;
-#pragma unroll
-  for (int c = 0; c < ProRegs<NT>::kPc; ++c) {
-    const int base = c * NT * 8 + tid * 8;
-    if (c < np) {
-      uint32_t lo = 0, hi = 0;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int32_t v = piece_get(X.pc[c], j);
-        const int32_t qm = min((abs(v) + half) >> e, 127);
-        const uint32_t b8 = (uint32_t)(uint8_t)(int8_t)(v < 0 ? -qm : qm);
-        if (j < 4) lo |= b8 << (8 * j);
-        else       hi |= b8 << (8 * (j - 4));
+      for (int i = 0; i < 4; ++i) {
+        const s16x2 v = as_s16x2(piece_word(X.pc[c], i));
+        hi = __builtin_elementwise_max(hi, v);
+        lo = __builtin_elementwise_min(lo, v);
       }
-      int t4 = __builtin_amdgcn_sdot4((int)lo, 0x01010101, 0, false);
+  int32_t mx = max(max((int)hi.x, (int)hi.y), -min((int)lo.x, (int)lo.y));
+  const int e = dynq8_exponent(red.max(wave_max_i32(mx), wave, lane));
+  // magnitudes in 16 bits: |x| <= 2^15, plus half (at most 2^8)
+  const unsigned short half = (unsigned short)((1 << e) >> 1), sh = (unsigned short)e;
+  const u16x2 halves = {half, half}, shifts = {sh, sh}, most = {127, 127};
+#pragma unroll
+  for (int c = 0; c < R::kPc; ++c)
+    if (c * NT * 8 < K) {
+      const int base = (c * NT + tid) * 8;
+      uint32_t q[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const s16x2 v = as_s16x2(piece_word(X.pc[c], i)), sg = v >> 15;
+        u16x2 m = __builtin_bit_cast(u16x2, (v ^ sg) - sg);
+        m = __builtin_elementwise_min((m + halves) >> shifts, most);
+        q[i] = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(s16x2, m) ^ sg) - sg);
+      }
+      const uint32_t lo8 = __builtin_amdgcn_perm(q[1], q[0], 0x06040200u);
+      const uint32_t hi8 = __builtin_amdgcn_perm(q[3], q[2], 0x06040200u);
+      int t4 = __builtin_amdgcn_sdot4((int)lo8, 0x01010101, 0, false);
       t4 += __builtin_amdgcn_update_dpp(0, t4, 0xB1, 0xF, 0xF, false);
       t4 += __builtin_amdgcn_update_dpp(0, t4, 0x4E, 0xF, 0xF, false);
       if (base < K) {
-        *(uint2 *)(xs + base) = make_uint2(lo, hi);
+        *(uint2 *)(xs + base) = make_uint2(lo8, hi8);
         if ((tid & 3) == 0) xlo[base / 32] = -8 * t4;
-        if (writer && P.x8_out) *(uint2 *)(P.x8_out + base) = make_uint2(lo, hi);
+        if (writer && P.x8_out) *(uint2 *)(P.x8_out + base) = make_uint2(lo8, hi8);
       }
     }
-  }
   if (writer && P.e_x_out && tid == 0) *P.e_x_out = e;
-  sync();
+  red.done(wave, lane);
   return e;
 }
 
 // ---------------------------------------------------------------------------
 // the GEMV: one 768-thread workgroup per CU, 3 teams of 4 wavefronts that
 // share one prologue.  Team v of workgroup r takes tiles r + G*(v + 3i);
-// its 4 wavefronts split a tile's scale blocks, each keeping its next block
-// in flight while it computes the current one.
+// its wavefronts split a tile's scale blocks, each keeping its next two
+// blocks in flight.  Where no workgroup has a second tile and a tile has more
+// than 4 blocks (a 4096 x 12288 down projection on 256 CUs), the 12
+// wavefronts are one team.  A tile's sums meet in an LDS slot; the wavefront
+// that adds last finishes the tile, so no team waits for another.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ const uint8_t *block_addr(const GemvParams &P, int tg, int b) {
   const int j = job_of(P, tg);
@@ -260,12 +383,12 @@ __device__ __forceinline__ const uint8_t *block_addr(const GemvParams &P, int tg
 }
 
 // This wavefront's blocks over the kernel: for its team's tiles it = 0, 1,
-// ... (tile r + G*(team + 3*it) < total_tiles), blocks b = wt, wt + 4, ...
-// < nblk -- nbw blocks per tile, the same for every tile.
+// ... (tile tg0 + VS * it < total_tiles), blocks b = wt, wt + W, ... < nblk --
+// nbw blocks per tile, the same for every tile.
 struct Item {
   int k;    // position in the sequence
   int it;   // tile iteration
-  int j;    // b = wt + 4j
+  int j;    // b = wt + W * j
 };
 __device__ __forceinline__ void item_next(Item &c, int nbw) {
   ++c.k;
@@ -305,94 +428,155 @@ __device__ __forceinline__ void issue_block(BlockRegs &R, const GemvParams &P, i
   issue_rsrc(R, block_rsrc(P, tg, b, real), lane);
 }
 
+// v is computed at this point
+__device__ __forceinline__ void computed(__amdgpu_buffer_rsrc_t rs) {
+  asm volatile("" ::"s"(rs));
+}
+// a copy of v that the compiler knows nothing about
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 constexpr int kGT = 768;
 constexpr int kGWaves = kGT / 64;
 constexpr int kGTeams = kGWaves / 4;
 constexpr int kPW0 = 4;                // teams 1 and 2 (wavefronts 4..11) run the prologue
 constexpr int kPT = kGT - 64 * kPW0;   // 512 threads
 
-// reduce a tile's 16 * p over the 4 k-quarter lanes and the team's 4
-// wavefronts, then round, check and write its 16 rows (one wavefront of the
-// team, rotating per tile)
-__device__ __forceinline__ void team_tile_finish(const GemvJob &J, int t, bool valid, int64_t p,
-                                                 int it, int team, int wt, int lane, int e_x,
-                                                 const uint16_t *sig, int32_t *err,
-                                                 int64_t (*red)[kGTeams][4][kTileRows],
-                                                 uint64_t &best) {
+// The LDS slots in which a team's tiles meet: tile `it` in slot it % kSlots.
+constexpr int kSlots = 8;
+struct TileSlot {
+  uint64_t sum[kTileRows];   // 16 * p of each row, zero between tiles
+  int32_t cnt;               // wavefronts that have added
+  int32_t gen;               // tiles the slot has finished
+};
+__device__ __forceinline__ void lds_add_u64(uint64_t *p, uint64_t v) {
+  asm volatile("ds_add_u64 %0, %1" :: "v"(lds_off(p)), "v"(v) : "memory");
+}
+__device__ __forceinline__ int32_t lds_add_rtn(int32_t *p, int32_t v) {
+  int32_t old;
+  asm volatile("ds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)"
+               : "=v"(old) : "v"(lds_off(p)), "v"(v) : "memory");
+  return old;
+}
+
+// 16 * p reduced over the 4 k-quarter lanes
+__device__ __forceinline__ int64_t quarter_sum(int64_t p) {
   p = (int64_t)((uint64_t)p + dpp_u64<0xB1, 0xF>((uint64_t)p));
-  p = (int64_t)((uint64_t)p + dpp_u64<0x4E, 0xF>((uint64_t)p));
-  const int par = it & 1;
-  if ((lane & 3) == 0) red[par][team][wt][lane >> 2] = p;
-  __syncthreads();
-  if (valid && wt == (it & 3) && lane < kTileRows) {
-    const int64_t tot = red[par][team][0][lane] + red[par][team][1][lane] +
-                        red[par][team][2][lane] + red[par][team][3][lane];
-    const int row = t * kTileRows + lane;
-    if (row < J.nrows) {
-      const int64_t y = rshr64(tot >> 4, J.sh);   // tot is 16 * p exactly
-      if (y > 2147483647LL || y < -2147483647LL) atomicOr(err, 1);
-      const int shift = J.p0 - e_x;
-      switch (J.epi) {
-        case EPI_Y32:
-          ((int32_t *)J.out)[row] = (int32_t)y;
-          break;
-        case EPI_MOVY_I16:
-          ((int16_t *)J.out)[row] = (int16_t)clamp64(movy_shift(y, shift), -32768, 32767);
-          break;
-        case EPI_MOVY_I16_ADD: {
-          const int64_t v = clamp64(movy_shift(y, shift), -32768, 32767);
-          if (J.out) ((int16_t *)J.out)[row] = (int16_t)v;
-          J.res_out[row] = (int16_t)clamp64(v + J.res[row], -32768, 32767);
-          break;
-        }
-        case EPI_MOVY_P32:
-          ((int32_t *)J.out)[row] =
-              (int32_t)clamp64(movy_shift(y, shift), -2147483648LL, 2147483647LL);
-          break;
-        case EPI_SILU32:
-          ((int16_t *)J.out)[row] = (int16_t)silu32(y, shift, sig);
-          break;
-        case EPI_SHIFT_I64:
-          ((int64_t *)J.out)[row] = movy_shift(y, shift);
-          break;
-        default: {   // EPI_ARGMAX: raw y32 (shift 0), seq_format.py:2225-2226
-          const uint64_t k = argmax_key((int32_t)y, (uint32_t)row);
-          best = k > best ? k : best;
-        }
+  return (int64_t)((uint64_t)p + dpp_u64<0x4E, 0xF>((uint64_t)p));
+}
+
+// Add this wavefront's share of a tile (quarter_sum) to the tile's slot; true in the wavefront that adds last of nw, which gets lane
+// l < 16's row sum in tot and leaves the slot free.  (A wavefront's LDS
+// instructions execute in order, so the count follows the sums.)
+__device__ __forceinline__ bool tile_add(TileSlot *slots, int it, int nw, int64_t p, int lane,
+                                         bool &ok, int64_t &tot) {
+  TileSlot &S = slots[it % kSlots];
+  // the tile that had the slot before is done (a wavefront is rarely 8 tiles
+  // ahead of its team)
+  if (it >= kSlots) ok = lds_wait_ge(&S.gen, it / kSlots) && ok;
+  if ((lane & 3) == 0) lds_add_u64(&S.sum[lane >> 2], (uint64_t)p);
+  int32_t old = 0;
+  if (lane == 0) old = lds_add_rtn(&S.cnt, 1);
+  if (__builtin_amdgcn_readfirstlane(old) != nw - 1) return false;
+  if (lane < kTileRows) {
+    tot = (int64_t)lds_read_u64(&S.sum[lane]);
+    lds_post_u64(&S.sum[lane], 0);
+  }
+  if (lane == 0) {
+    lds_post_i32(&S.cnt, 0);
+    lds_post_i32(&S.gen, it / kSlots + 1);
+  }
+  return true;
+}
+
+// round, check and write the 16 rows of tile t (lane l: row 16 t + l)
+__device__ __forceinline__ void tile_finish(const GemvJob &J, int t, int64_t tot, int lane,
+                                            int e_x, const uint16_t *sig, int32_t *err,
+                                            uint64_t &best) {
+  const int row = t * kTileRows + lane;
+  if (lane < kTileRows && row < J.nrows) {
+    const int64_t y = rshr64(tot >> 4, J.sh);   // tot is 16 * p exactly
+    if (y > 2147483647LL || y < -2147483647LL) atomicOr(err, 1);
+    const int shift = J.p0 - e_x;
+    switch (J.epi) {
+      case EPI_Y32:
+        ((int32_t *)J.out)[row] = (int32_t)y;
+        break;
+      case EPI_MOVY_I16:
+        ((int16_t *)J.out)[row] = (int16_t)clamp64(movy_shift(y, shift), -32768, 32767);
+        break;
+      case EPI_MOVY_I16_ADD: {
+        const int64_t v = clamp64(movy_shift(y, shift), -32768, 32767);
+        if (J.out) ((int16_t *)J.out)[row] = (int16_t)v;
+        J.res_out[row] = (int16_t)clamp64(v + J.res[row], -32768, 32767);
+        break;
+      }
+      case EPI_MOVY_P32:
+        ((int32_t *)J.out)[row] =
+            (int32_t)clamp64(movy_shift(y, shift), -2147483648LL, 2147483647LL);
+        break;
+      case EPI_SILU32:
+        ((int16_t *)J.out)[row] = (int16_t)silu32(y, shift, sig);
+        break;
+      case EPI_SHIFT_I64:
+        ((int64_t *)J.out)[row] = movy_shift(y, shift);
+        break;
+      default: {   // EPI_ARGMAX: raw y32 (shift 0), seq_format.py:2225-2226
+        const uint64_t k = argmax_key((int32_t)y, (uint32_t)row);
+        best = k > best ? k : best;
       }
     }
   }
 }
 
+template <int PRO>
 __global__ __launch_bounds__(kGT) void gemv_kernel(GemvParams P) {
   __shared__ __align__(16) int8_t xs[kKMax];
   __shared__ int32_t xlo[kKMax / 32];
-  __shared__ int64_t red[2][kGTeams][4][kTileRows];
-  __shared__ int64_t sm[2 * kGWaves];
+  __shared__ TileSlot slots[kGTeams][kSlots];
+  __shared__ int64_t red[2][kGTeams][4][kTileRows];   // lockstep
   __shared__ uint64_t keys[kGWaves];
-  __shared__ uint16_t tab_rsqrt[512], tab_sig[264];
-  __shared__ int32_t tsync[16];   // prologue group's phases [0, 8), done [8], e_x [9]
+  __shared__ uint16_t tab_rsqrt[PRO == PRO_RMSNORM_DYNQ8 ? 512 : 1], tab_sig[264];
+  __shared__ ProWords words;
 
-  const int tid = threadIdx.x, lane = tid & 63, q = lane & 3;
+  const int tid = threadIdx.x, lane = tid & 63;
   // wave index as a scalar so the block loops below branch on SGPRs
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int team = wave >> 2, wt = wave & 3;
   const int NG = P.NG, nblk = P.nblk, T = P.total_tiles;
-  const int G = gridDim.x, r = blockIdx.x, VS = G * kGTeams;
-  if (tid < 16) tsync[tid] = 0;
+  const int G = gridDim.x, r = blockIdx.x;
+  // one team of 12: 4096 x 12288 8.4 -> 6.4 us from the first workgroup's start
+  // to the last's end (a tile's 24 blocks on 12 wavefronts, two each, instead
+  // of six in turn on four)
+  const bool wide = T <= G && nblk > 4;
+  const int W = wide ? kGWaves : 4;                 // wavefronts of a team
+  const int team = wide ? 0 : wave >> 2, wt = wide ? wave : wave & 3;
+  const int VS = wide ? G : G * kGTeams;
+  const int nw = min(W, nblk);                      // ... that have blocks of a tile
+  if (tid < (int)(sizeof(words) / 4)) ((int32_t *)&words)[tid] = 0;
+  for (int i = tid; i < (int)(sizeof(slots) / 4); i += kGT) ((int32_t *)slots)[i] = 0;
+  // A long stream (the LM head) keeps its wavefronts in step, one barrier per
+  // tile iteration: the GPU then sweeps one window of memory, where drifting
+  // wavefronts read at 0.92 of that (248,320 x 4096: 81.3 us in step, 89 us
+  // without).  Short launches (up to two tiles per team) run without: no team
+  // waits for another's first blocks (chained step in graph mode 1.33 ms in
+  // step from the second tile on, 1.29 ms without).
+  const bool lockstep = T > 2 * VS;
+  if (lockstep)
+    for (int i = tid; i < (int)(sizeof(red) / 4); i += kGT) ((int32_t *)red)[i] = 0;
 
   // A CU's first weight blocks take microseconds to drain at its share of
   // HBM bandwidth, and a wavefront cannot issue past a load the memory
-  // pipeline has no room for.  So teams 1 and 2 run the prologue alone,
-  // with their own LDS barrier: they issue the activation and table loads,
-  // the workgroup meets once (nothing is waited for), and only then does
-  // team 0 put its first blocks in flight, behind the activations.  Team 0
-  // waits for the prologue's result; teams 1 and 2 start their blocks after
-  // it.
+  // pipeline has no room for.  So teams 1 and 2 issue the activation and
+  // table loads, the workgroup meets once (nothing is waited for), and only
+  // then do wavefronts 0-3 put their first blocks in flight, behind the
+  // activations.  Wavefronts 4-11 issue theirs after the prologue: issued
+  // before its arithmetic, they stall it for as long as the memory pipeline is
+  // full (chained step in graph mode 1.44 -> 1.61 ms).
   // Two register sets per wavefront, A and B, hold its next two blocks.
-  // Team 0 puts both in flight at once; teams 1 and 2 after the prologue.
   const int tg0 = r + G * team;
-  const int nbw = wt < nblk ? (nblk - wt + 3) / 4 : 0;
+  const int nbw = wt >= nblk ? 0 : wide ? (nblk - wt + kGWaves - 1) / kGWaves : (nblk - wt + 3) / 4;
   const int nitems = tg0 < T ? ((T - 1 - tg0) / VS + 1) * nbw : 0;
   Item ca{0, 0, 0}, cb = ca;
   if (nbw > 0) item_next(cb, nbw);
@@ -400,87 +584,98 @@ __global__ __launch_bounds__(kGT) void gemv_kernel(GemvParams P) {
   if (nbw > 0) item_next(cn, nbw);
   BlockRegs A, B;
   const int pt = tid - kPW0 * 64;   // thread index within the prologue group
+  GroupRed grp{&words, true};
   int e_x;
-  bool ok;
-  if (team == 0) {
-    // the blocks' addresses first (the kernel arguments they need come in
-    // by scalar loads, a round trip or two at a launch's start), so that
-    // the loads go out as soon as the workgroup has met: C0 as one launch
-    // per matrix 5.49 -> 5.38 us
+  if (wave < kPW0) {
+    // the blocks' addresses first (the kernel arguments they need come in by
+    // scalar loads, a round trip or two at a launch's start), so that the
+    // loads go out as soon as the workgroup has met: C0 as one launch per
+    // matrix 5.49 -> 5.38 us
     const __amdgpu_buffer_rsrc_t rsA = block_rsrc(P, tg0, wt, nitems > 0);
     const __amdgpu_buffer_rsrc_t rsB =
-        block_rsrc(P, tg0 + VS * cb.it, wt + 4 * cb.j, cb.k < nitems);
-    asm volatile("" ::"s"(rsA), "s"(rsB));
-    __syncthreads();
+        block_rsrc(P, tg0 + VS * cb.it, wt + W * cb.j, cb.k < nitems);
+    computed(rsA);
+    computed(rsB);
+    meet();
     issue_rsrc(A, rsA, lane);
     issue_rsrc(B, rsB, lane);
-    ok = lds_wait_ge(&tsync[8], 1);
-    e_x = lds_read_i32(&tsync[9]);
+    grp.wait_ready<true>(lane);
+    e_x = PRO == PRO_X8 ? P.e_x_given : dynq8_exponent(grp.all_max(lane));
+    e_x = __builtin_amdgcn_readfirstlane(e_x);
   } else {
     static_assert(kPT >= 512 && kPT >= 257, "one table entry per thread");
-    const int trs = P.tables[kRsqrtOff + (pt < 512 ? pt : 0)];
+    ProRegs<PRO, kPT> X;
+    pro_load<PRO, kPT>(P, X, pt);
+    int trs = 0;
+    if constexpr (PRO == PRO_RMSNORM_DYNQ8) trs = P.tables[kRsqrtOff + pt];
     const int tsg = P.tables[kSigmoidOff + (pt < 257 ? pt : 0)];
-    ProRegs<kPT> X;
-    pro_load<kPT>(P, X, pt);
-    __syncthreads();
-    if (pt < 512) tab_rsqrt[pt] = (uint16_t)trs;
+    meet();
+    if constexpr (PRO == PRO_RMSNORM_DYNQ8) tab_rsqrt[pt] = (uint16_t)trs;
     if (pt < 257) tab_sig[pt] = (uint16_t)tsg;
-    GroupSync<kPT / 64> sync{tsync, kPW0, 0, true};
-    e_x = pro_compute<kPT>(P, X, xs, xlo, sm, tab_rsqrt, pt, sync);
-    ok = sync.ok;
-    // every LDS write of the group is complete (its last barrier): publish
-    if (pt == 0) {
-      lds_write_i32(&tsync[9], e_x);
-      lds_write_i32(&tsync[8], 1);
+    e_x = pro_compute<PRO, kPT>(P, X, xs, xlo, tab_rsqrt, pt, grp);
+    e_x = __builtin_amdgcn_readfirstlane(e_x);
+    if (nitems > 0) {
+      issue_block(A, P, tg0, wt, true, lane);
+      issue_block(B, P, tg0 + VS * cb.it, wt + W * cb.j, cb.k < nitems, lane);
     }
-    issue_block(A, P, tg0, wt, nitems > 0, lane);
-    issue_block(B, P, tg0 + VS * cb.it, wt + 4 * cb.j, cb.k < nitems, lane);
   }
 
+  // the first tile's job, its fields read before anything waits for them
+  int jcur = job_of(P, tg0 < T ? tg0 : 0);
+  GemvJob J = P.job[jcur];
   const uint16_t *sig = tab_sig;
   uint64_t best = 0;   // argmax key (0 == none)
-  // every team runs the same number of tile iterations (the reductions
-  // inside are workgroup barriers); team 0 has the most tiles
-  const int iters = T > r ? (T - r + VS - 1) / VS : 0;
-  int fin = 0;   // tile iterations finished
   int64_t p = 0;
-  // consume the block in R (item c), finish its tile after the wavefront's
+  int fin = 0;   // lockstep: tile iterations finished
+  // consume the block in R (item c), add to its tile after the wavefront's
   // last block of it, and refill R with the item two ahead
   auto step = [&](BlockRegs &R, Item &c) {
     // lane-derived offsets are recomputed from an opaque copy of the thread
     // index, so the compiler does not keep them all live across the loop
-    int tid_s = tid;
-    asm volatile("" : "+v"(tid_s));
+    const int tid_s = opaque(tid);
     const int lane = tid_s & 63, q = lane & 3;
-    const int b = wt + 4 * c.j;
-    const int tg = tg0 + VS * c.it;
+    const int b = wt + W * c.j;
+    const int tg = tg0 + VS * c.it, it = c.it;
+    const bool last = c.j == nbw - 1;
     p = dot_block(R, groups_in(NG, b), b * kGroupsPerBlock, q, xs, xlo, p);
-    if (c.j == nbw - 1) {
-      const GemvJob &J = P.job[job_of(P, tg)];
-      team_tile_finish(J, tg - J.tile0, true, p, fin, team, wt, lane, e_x, sig, P.err, red,
-                       best);
-      ++fin;
+    if (last) {
+      p = quarter_sum(p);
+      int64_t tot = 0;
+      bool mine;
+      if (lockstep) {
+        if ((lane & 3) == 0) red[it & 1][team][wt][lane >> 2] = p;
+        meet();
+        ++fin;
+        mine = wt == it % nw;
+        if (mine)
+          tot = red[it & 1][team][0][lane & 15] + red[it & 1][team][1][lane & 15] +
+                red[it & 1][team][2][lane & 15] + red[it & 1][team][3][lane & 15];
+      } else {
+        mine = tile_add(slots[team], it, nw, p, lane, grp.ok, tot);
+      }
+      if (mine) {
+        const int j = job_of(P, tg);
+        if (j != jcur) {
+          jcur = j;
+          J = P.job[j];
+        }
+        tile_finish(J, tg - J.tile0, tot, lane, e_x, sig, P.err, best);
+      }
       p = 0;
     }
     c = cn;
     item_next(cn, nbw);
-    issue_block(R, P, tg0 + VS * c.it, wt + 4 * c.j, c.k < nitems, lane);
+    issue_block(R, P, tg0 + VS * c.it, wt + W * c.j, c.k < nitems, lane);
   };
   for (int k = 0; k < nitems; k += 2) {
     step(A, ca);
     if (k + 1 >= nitems) break;
     step(B, cb);
   }
-  // tiles this wavefront has no block of: it still takes part in the
-  // team's reduction, and is the writer of every fourth
-  for (; fin < iters; ++fin) {
-    const int tg = tg0 + VS * fin;
-    const bool valid = tg < T;
-    const GemvJob &J = P.job[job_of(P, valid ? tg : 0)];
-    team_tile_finish(J, valid ? tg - J.tile0 : 0, valid, 0, fin, team, wt, lane, e_x, sig,
-                     P.err, red, best);
-  }
-  if (!ok && lane == 0) atomicOr(P.err, 4);
+  // tile iterations this wavefront has no block of (team 0 has the most tiles)
+  if (lockstep)
+    for (const int iters = (T - r + VS - 1) / VS; fin < iters; ++fin) meet();
+  if (!grp.ok && lane == 0) atomicOr(P.err, 4);
   if (P.partials) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -518,14 +713,15 @@ __global__ __launch_bounds__(kWG) void argmax_final_kernel(
 }
 
 // prologue only: DYNQ8 / RMSNorm(+DYNQ8) of one vector, one workgroup
+template <int PRO>
 __global__ __launch_bounds__(kWG) void vec_prologue_kernel(GemvParams P) {
   __shared__ __align__(16) int8_t xs[kKMax];
   __shared__ int32_t xlo[kKMax / 32];
   __shared__ int64_t sm[2 * kWaves];
-  ProRegs<kWG> X;
-  pro_load<kWG>(P, X, threadIdx.x);
-  WgSync sync;
-  pro_compute<kWG>(P, X, xs, xlo, sm, P.tables + kRsqrtOff, threadIdx.x, sync);
+  ProRegs<PRO, kWG> X;
+  pro_load<PRO, kWG>(P, X, threadIdx.x);
+  WgRed<kWaves> red{sm};
+  pro_compute<PRO, kWG>(P, X, xs, xlo, P.tables + kRsqrtOff, threadIdx.x, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -761,14 +957,45 @@ hipError_t launch_unpack(const uint8_t *src, int64_t nrows, const Layout &L,
   return hipGetLastError();
 }
 
-hipError_t launch_gemv(const GemvParams &p, int grid, hipStream_t s) {
-  hipLaunchKernelGGL(gemv_kernel, dim3(grid), dim3(kGT), 0, s, p);
+hipError_t launch_gemv_timed(const GemvParams &p, int grid, hipStream_t s,
+                             hipEvent_t start, hipEvent_t stop) {
+  const dim3 g(grid), b(kGT);
+  switch (p.pro) {
+    case PRO_X8:
+      hipExtLaunchKernelGGL(gemv_kernel<PRO_X8>, g, b, 0, s, start, stop, 0, p);
+      break;
+    case PRO_DYNQ8:
+      hipExtLaunchKernelGGL(gemv_kernel<PRO_DYNQ8>, g, b, 0, s, start, stop, 0, p);
+      break;
+    case PRO_RMSNORM_DYNQ8:
+      hipExtLaunchKernelGGL(gemv_kernel<PRO_RMSNORM_DYNQ8>, g, b, 0, s, start, stop, 0, p);
+      break;
+    case PRO_EMUL_DYNQ8:
+      hipExtLaunchKernelGGL(gemv_kernel<PRO_EMUL_DYNQ8>, g, b, 0, s, start, stop, 0, p);
+      break;
+    default:
+      return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_gemv_timed(const GemvParams &p, int grid, hipStream_t s,
-                             hipEvent_t start, hipEvent_t stop) {
-  hipExtLaunchKernelGGL(gemv_kernel, dim3(grid), dim3(kGT), 0, s, start, stop, 0, p);
+hipError_t launch_gemv(const GemvParams &p, int grid, hipStream_t s) {
+  switch (p.pro) {
+    case PRO_X8:
+      hipLaunchKernelGGL(gemv_kernel<PRO_X8>, dim3(grid), dim3(kGT), 0, s, p);
+      break;
+    case PRO_DYNQ8:
+      hipLaunchKernelGGL(gemv_kernel<PRO_DYNQ8>, dim3(grid), dim3(kGT), 0, s, p);
+      break;
+    case PRO_RMSNORM_DYNQ8:
+      hipLaunchKernelGGL(gemv_kernel<PRO_RMSNORM_DYNQ8>, dim3(grid), dim3(kGT), 0, s, p);
+      break;
+    case PRO_EMUL_DYNQ8:
+      hipLaunchKernelGGL(gemv_kernel<PRO_EMUL_DYNQ8>, dim3(grid), dim3(kGT), 0, s, p);
+      break;
+    default:
+      return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
@@ -781,7 +1008,10 @@ hipError_t launch_argmax_final(const uint64_t *partials, int n, int32_t *result,
 }
 
 hipError_t launch_vec_prologue(const GemvParams &p, hipStream_t s) {
-  hipLaunchKernelGGL(vec_prologue_kernel, dim3(1), dim3(kWG), 0, s, p);
+  if (p.pro == PRO_RMSNORM_DYNQ8)
+    hipLaunchKernelGGL(vec_prologue_kernel<PRO_RMSNORM_DYNQ8>, dim3(1), dim3(kWG), 0, s, p);
+  else
+    hipLaunchKernelGGL(vec_prologue_kernel<PRO_DYNQ8>, dim3(1), dim3(kWG), 0, s, p);
   return hipGetLastError();
 }
 
@@ -829,7 +1059,7 @@ hipError_t launch_alu(int op, const int32_t *y, const int16_t *b, int64_t n, int
 
 int gemv_max_blocks_per_cu() {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemv_kernel, kGT, 0) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, gemv_kernel<PRO_DYNQ8>, kGT, 0) !=
           hipSuccess || n < 1)
     n = 1;
   return n;
