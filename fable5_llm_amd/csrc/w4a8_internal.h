@@ -165,6 +165,20 @@ hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t s);
 // stop (optional) are recorded by the dispatch itself
 hipError_t launch_read(const void *buf, int64_t nbytes, uint32_t *sink, int grid,
                        hipStream_t s, hipEvent_t start, hipEvent_t stop);
+// Copies between pinned host memory and device memory in one launch, for the
+// host-buffer entry points: n bytes (a multiple of 16) from src to dst, then
+// (flag set) *err_out = *err and, once all of it is visible to the host,
+// *flag = seq.  All addresses are the device's; 16-byte aligned.
+struct HostCopy {
+  const void *src;
+  void *dst;
+  int32_t n;
+  const int32_t *err;
+  int32_t *err_out;
+  uint32_t *flag;
+  uint32_t seq;
+};
+hipError_t launch_host_copy(const HostCopy &c, hipStream_t s);
 hipError_t launch_repack(const uint8_t *img, int64_t nrows, const Layout &L,
                          int64_t stride, uint8_t *dst, hipStream_t s);
 hipError_t launch_unpack(const uint8_t *src, int64_t nrows, const Layout &L,

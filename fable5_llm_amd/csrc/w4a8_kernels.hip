@@ -843,6 +843,21 @@ __global__ void fill_i32_kernel(int32_t *p, int32_t v, int64_t n) {
     p[i] = v;
 }
 
+// One workgroup: the copies are a few KB to 150 KB, and a single group can
+// tell when all of it has been written.  Bound by the link's round trip.
+__global__ __launch_bounds__(1024) void host_copy_kernel(HostCopy c) {
+  const uint4 *src = (const uint4 *)c.src;
+  uint4 *dst = (uint4 *)c.dst;
+  const int n16 = c.n / 16;
+  for (int i = threadIdx.x; i < n16; i += 1024) dst[i] = src[i];
+  if (!c.flag) return;
+  if (threadIdx.x == 0) *c.err_out = *c.err;
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(c.flag, c.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void rshift_round_kernel(const int64_t *v, int64_t n, int s, int64_t *out) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
@@ -929,6 +944,11 @@ hipError_t launch_read(const void *buf, int64_t nbytes, uint32_t *sink, int grid
 hipError_t launch_fill_i32(int32_t *p, int32_t v, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(fill_i32_kernel, dim3(blocks_for(n, 256, 4096)), dim3(256),
                      0, s, p, v, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_host_copy(const HostCopy &c, hipStream_t s) {
+  hipLaunchKernelGGL(host_copy_kernel, dim3(1), dim3(1024), 0, s, c);
   return hipGetLastError();
 }
 

@@ -6,6 +6,7 @@ Host-array methods (numpy in, numpy out) are synchronous; *_async methods
 take torch tensors already on the device and enqueue on the context stream.
 """
 import ctypes
+from array import array
 
 import numpy as np
 
@@ -15,12 +16,23 @@ _c = ctypes.c_void_p
 
 
 def _ptr(a):
-    return ctypes.c_void_p(a.ctypes.data)
+    """address of a numpy array's data"""
+    return a.__array_interface__["data"][0]
 
 
 def _dptr(t):
     """device pointer of a torch tensor (or None)"""
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+def _i32s(values):
+    """int32 array of a sequence of whole numbers (OverflowError outside
+    int32)"""
+    return array("i", [int(v) for v in values])
+
+
+def _aptr(a):
+    return a.buffer_info()[0]
 
 
 def _dev(t, need_bytes, name, required=True):
@@ -32,6 +44,11 @@ def _dev(t, need_bytes, name, required=True):
         if required:
             raise ValueError(f"{name}: a device tensor is required")
         return
+    try:
+        if t.is_cuda and t.nbytes >= need_bytes and t.is_contiguous():
+            return
+    except AttributeError:
+        pass
     if not getattr(t, "is_cuda", False):
         raise ValueError(f"{name}: must be a device tensor")
     if not t.is_contiguous():
@@ -338,10 +355,9 @@ class Context:
         _dev(xn_out, 2 * K, "xn_out", required=False)
         wa = (ctypes.c_void_p * n)(*[w.h.value for w in weights])
         oa = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
-        ea = np.ascontiguousarray(epilogues, dtype=np.int32)
-        pa = np.ascontiguousarray(p0s, dtype=np.int32)
+        ea, pa = _i32s(epilogues), _i32s(p0s)
         N.check(N.lib().w4a8_site_async(
-            self.h, n, wa, _ptr(ea), _ptr(pa), oa, int(prologue), _dptr(x),
+            self.h, n, wa, _aptr(ea), _aptr(pa), oa, int(prologue), _dptr(x),
             _dptr(norm_w), int(in_f), 1 if one_plus else 0, int(e_x), _dptr(x8_out),
             _dptr(e_x_out), _dptr(xn_out)), "site")
 
@@ -436,10 +452,9 @@ class Plan:
         _dev(xn_out, 2 * K, "xn_out", required=False)
         wa = (ctypes.c_void_p * n)(*[w.h.value for w in weights])
         oa = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
-        ea = np.ascontiguousarray(epilogues, dtype=np.int32)
-        pa = np.ascontiguousarray(p0s, dtype=np.int32)
+        ea, pa = _i32s(epilogues), _i32s(p0s)
         N.check(N.lib().w4a8_plan_add_site(
-            self.h, n, wa, _ptr(ea), _ptr(pa), oa, int(prologue), _dptr(x),
+            self.h, n, wa, _aptr(ea), _aptr(pa), oa, int(prologue), _dptr(x),
             _dptr(norm_w), int(in_f), 1 if one_plus else 0, int(e_x),
             _dptr(x8_out), _dptr(e_x_out), _dptr(xn_out)), "plan_add_site")
         self._keep += [weights, outs, x, norm_w, x8_out, e_x_out, xn_out]
@@ -464,10 +479,9 @@ class Plan:
         _dev(e_x_out, 4, "e_x_out", required=False)
         wa = (ctypes.c_void_p * n)(*[w.h.value for w in weights])
         oa = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
-        ea = np.ascontiguousarray(epilogues, dtype=np.int32)
-        pa = np.ascontiguousarray(p0s, dtype=np.int32)
+        ea, pa = _i32s(epilogues), _i32s(p0s)
         N.check(N.lib().w4a8_plan_add_site_emul(
-            self.h, n, wa, _ptr(ea), _ptr(pa), oa, _dptr(x), _dptr(x2),
+            self.h, n, wa, _aptr(ea), _aptr(pa), oa, _dptr(x), _dptr(x2),
             _dptr(x8_out), _dptr(e_x_out)), "plan_add_site_emul")
         self._keep += [weights, outs, x, x2, x8_out, e_x_out]
         self.bytes += sum(w.wire_bytes for w in weights)
