@@ -295,7 +295,7 @@ hipError_t launch_matmul_multi(const MmJobSpec *jobs, int n, int32_t B, int32_t 
 // matmul_plan_prepare writes on the host, with the launch shape in cfg.
 constexpr int kMmPlanJobs = 128;
 struct MmPlanCfg {
-  int32_t B, CT, TM, KS, units, wgs;
+  int32_t B, CT, TM, KS, NW, units, wgs;
 };
 hipError_t matmul_plan_prepare(const MmJobSpec *jobs, int n, int32_t B,
                                std::vector<uint8_t> &table, MmPlanCfg *cfg);

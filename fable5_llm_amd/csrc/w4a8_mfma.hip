@@ -13,7 +13,8 @@
 // v_mad_i64_i32, which runs at the rate of a double-precision FMA (measured:
 // 2.4 against 2.2 ns per instruction and SIMD) and needs no conversion.
 //
-// Four wavefronts per workgroup, two workgroups per CU.  What bounds it is the
+// Four wavefronts per workgroup, two workgroups per CU (or one of eight
+// wavefronts).  What bounds it is the
 // weight stream, and next to it the activations: 16 tokens of a group are
 // 2 KiB for every KiB of weights they meet.  Loaded straight into the MFMA's
 // layout they touch 16 cache lines per 16 lanes, and the address unit takes
@@ -23,8 +24,8 @@
 // unit (up to TM tiles per wavefront, all of K) over the wavefronts:
 //
 //  * shared (KS = 1): every wavefront takes its own TM tiles and all of K, and
-//    the four share one copy of the activations (one workgroup barrier per
-//    four groups).  Nothing is reduced; best where tiles are plenty.
+//    all four or eight share one copy of the activations (one workgroup
+//    barrier per four groups).  Nothing is reduced; best where tiles are plenty.
 //  * split (KS = 4): the wavefronts take the same tile and every fourth quad
 //    of groups, each with its own copies (no barrier), and meet in an LDS
 //    table at the end of the unit.
@@ -33,15 +34,15 @@
 // wavefront) and the copies run on across them, so the stream does not drain
 // between tiles or matrices.  No wait depends on another workgroup.
 //
-// Measured, cold weights (us per launch, before: one workgroup per CU with
-// loader wavefronts and 8 slots, which waited for each slot's copies in turn):
-//   12288 + 12288 rows, K 4096:  B = 8: 19.0 -> 14.0, B = 64: 100 -> 21
-//   4096 rows, K 12288:          B = 8: 12.8 -> 10.2, B = 64: 52 -> 19
-//   60,000 rows, K 4096:         B = 8: 32 -> 25, B = 32: 50 -> 30, B = 64: 241 -> 40
-//   a pass of 96 FFN matrices:   B = 8: 534 -> 464, B = 32: 711 -> 565, B = 64: 4040 -> 680
-// (the pass's weights alone take 360 us at the read ceiling).  The 117 MB
-// of y32 that a pass writes at B = 32 cost 55 us of it (a copy that stores
-// nothing), the rest is the activations' way through L1 and LDS.
+// Measured, cold weights, us per launch: with a scale load per group and four
+// wavefronts everywhere -> now (a pass took 534, 711 and 4040 us with one
+// workgroup per CU, loader wavefronts and 8 slots):
+//   12288 + 12288 rows, K 4096:  B = 8: 13.7 -> 13.3, B = 64: 21.1 -> 18.6
+//   4096 rows, K 12288:          B = 8: 8.8 -> 8.6, B = 64: 19.2 -> 18.4
+//   60,000 rows, K 4096:         B = 8: 25.7 -> 23.9, B = 32: 29.4 -> 26.0, B = 64: 36.7 -> 32.8
+//   a pass of 96 FFN matrices:   B = 8: 430 -> 402, B = 32: 531 -> 457, B = 64: 625 -> 537
+// The pass's weights alone take 360 us at the read ceiling; the 117 MB of y32
+// that it writes at B = 32 take about 50 us of the rest.
 #include <algorithm>
 
 #include "w4a8_device.h"
@@ -57,7 +58,7 @@ constexpr int kMAuxNt = 2;                 // buffer-load cache policy: non-temp
 constexpr int kMPast = 0x40000000;         // a buffer offset past every range
 constexpr int kLdsBytes = 160 * 1024;
 constexpr int kMWaves = 4;
-constexpr int kMThreads = 64 * kMWaves;
+constexpr int kMWide = 8;                  // wavefronts of a wide shared workgroup
 
 // A unit: up to TM * TS consecutive row tiles of one matrix, over all of K.
 struct MmUnit {
@@ -94,6 +95,7 @@ __device__ __forceinline__ int cvt_hi16(uint32_t w) {
 }
 
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const void *p, int bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, bytes, kMBufDword3);
@@ -179,22 +181,26 @@ constexpr size_t mm_x_bytes(int CT, int KS, bool half8) {
 
 // half8: at most 8 tokens (one octet is copied, and read by both halves of
 // the MFMA's 16 rows)
-template <int TM, int CT, int KS, bool half8, bool plan>
-__global__ __launch_bounds__(kMThreads, 2) void matmul_kernel(MmParams P) {
+template <int NW, int TM, int CT, int KS, bool half8, bool plan>
+__global__ __launch_bounds__(64 * NW, 2) void matmul_kernel(MmParams P) {
   extern __shared__ __align__(1024) uint8_t smem[];
-  constexpr int NW = kMWaves, TS = NW / KS;
+  constexpr int TS = NW / KS;
   constexpr int Q = mm_q(CT, KS), NBUF = mm_nbuf(CT, KS);
   constexpr int NO = mm_octets(CT, half8);
   constexpr int kGrp = NO * 1024;                   // LDS bytes of a group's activations
   constexpr int kBuf = Q * kGrp;                    // ... of a step
   constexpr int ND = TS == 1 ? Q * NO : Q * NO / NW;   // copies per wavefront and step
-  constexpr int D = 4;                              // groups in flight
+  constexpr int D = 4;                           // groups in flight
   constexpr int kTurn = KS * D;                     // groups of a turn of the ring, all slices
   constexpr int kXBytes = (int)mm_x_bytes(CT, KS, half8);
+  // the scales' 256 bytes of a block are read twice, half a block apart: kept
+  // in the cache, except beyond 48 tokens, where the activations need it more
+  // (96 FFN matrices: B = 32 493 us non-temporal, 477 not; B = 64 586 and 598)
+  constexpr int kMAuxM = CT == 4 ? kMAuxNt : 0;
   constexpr int NR = TM * CT * 4 * 64;              // a wavefront's sums
   static_assert(KS == 1 || KS == NW, "the copies are shared by all wavefronts or by none");
   static_assert(ND * 1024 * (TS == 1 ? 1 : NW) == kBuf, "whole copies per wavefront");
-  static_assert(NBUF - 1 < D / Q || NBUF == 2, "a step's copies reach one turn ahead at most");
+  static_assert(NBUF - 1 <= D / Q || NBUF == 2, "a step's copies reach one turn ahead at most");
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ks = TS == 1 ? wave : 0, ts = TS == 1 ? 0 : wave;
@@ -246,18 +252,20 @@ __global__ __launch_bounds__(kMThreads, 2) void matmul_kernel(MmParams P) {
   };
   const int wlane = kScaleChunk + (c * 4 + q) * 16, slane = c * 16;
   u4 w[TM][D];
-  uint32_t m[TM][D];
+  // the turn's scales and the next turn's, a lane's four groups in one load
+  // (a load per group and tile, 2 bytes a lane: B = 8 432 us, 423 so)
+  u2 m[TM], mn[TM];
   auto load_w = [&](const MmSrc &S, int g, const int slot) {
     const int off = (g >> 3) * kBlockBytes + (g & 7) * kGroupChunk + wlane;
 #pragma unroll
     for (int j = 0; j < TM; ++j)
       w[j][slot] = __builtin_amdgcn_raw_buffer_load_b128(mm_tile_rsrc(S, j), off, 0, kMAuxNt);
   };
-  auto load_m = [&](const MmSrc &S, int g, const int slot) {
-    const int off = (g >> 3) * kBlockBytes + (g & 7) * 2 + slane;
+  auto load_m = [&](const MmSrc &S, int g) {
+    const int off = (g >> 3) * kBlockBytes + (g & 7) * 2 + slane;   // g: a multiple of 4
 #pragma unroll
     for (int j = 0; j < TM; ++j)
-      m[j][slot] = __builtin_amdgcn_raw_buffer_load_b16(mm_tile_rsrc(S, j), off, 0, kMAuxNt);
+      mn[j] = __builtin_amdgcn_raw_buffer_load_b64(mm_tile_rsrc(S, j), off, 0, kMAuxM);
   };
 
   int64_t p[TM][CT][4];
@@ -276,17 +284,17 @@ __global__ __launch_bounds__(kMThreads, 2) void matmul_kernel(MmParams P) {
     wait_lds();
     __builtin_amdgcn_s_barrier();
   }
+  load_m(S, ks * D);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int s = 0; s < NBUF - 1; ++s) copy_x(S, s / (D / Q) * kTurn + s % (D / Q) * Q, s);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < D; ++i) {
     load_w(S, ks * D + i, i);
-    load_m(S, ks * D + i, i);
-    __builtin_amdgcn_sched_barrier(0);
   }
   // the first step's activations: everything issued after them may be in flight
-  mm_wait_vm<(NBUF - 2) * ND + 2 * TM * D>();
+  mm_wait_vm<(NBUF - 2) * ND + TM * D>();
   if constexpr (TS > 1) __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
 
@@ -301,6 +309,10 @@ __global__ __launch_bounds__(kMThreads, 2) void matmul_kernel(MmParams P) {
       const bool last = g0 + kTurn >= U.NG;
       const MmSrc T = last ? src_of(V) : S;      // the next turn's loads
       const int gt = last ? 0 : g0 + kTurn;
+#pragma unroll
+      for (int j = 0; j < TM; ++j) m[j] = mn[j];
+      load_m(T, gt + ks * D);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < D; ++i) {
         if (i % Q == 0) {
@@ -335,7 +347,7 @@ __global__ __launch_bounds__(kMThreads, 2) void matmul_kernel(MmParams P) {
 #pragma unroll
         for (int j = 0; j < TM; ++j) {
           // opaque, so that the compiler forms 32 x 32 + 64 signed multiply-adds
-          const int32_t mv = mm_opaque((int32_t)m[j][i]);
+          const int32_t mv = mm_opaque((int32_t)(i & 1 ? m[j][i / 2] >> 16 : m[j][i / 2] & 0xFFFFu));
 #pragma unroll
           for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -343,11 +355,9 @@ __global__ __launch_bounds__(kMThreads, 2) void matmul_kernel(MmParams P) {
               p[j][ct][e] += (int64_t)mv * (int64_t)acc[j][ct][e];
         }
         __builtin_amdgcn_sched_barrier(0);
-        load_m(T, gt + ks * D + i, i);
-        __builtin_amdgcn_sched_barrier(0);
         if (i % Q == Q - 1) {
           // the next step's activations: issued NBUF - 1 steps ago
-          mm_wait_vm<(NBUF - 2) * (ND + 2 * TM * Q) + 2 * TM * Q>();
+          mm_wait_vm<(NBUF - 2) * (ND + TM * Q) + TM * Q>();
           if constexpr (TS > 1) __builtin_amdgcn_s_barrier();
           __builtin_amdgcn_sched_barrier(0);
           buf = buf + 1 == NBUF ? 0 : buf + 1;
@@ -414,13 +424,13 @@ __global__ __launch_bounds__(kMThreads, 2) void matmul_kernel(MmParams P) {
   if (ovf) atomicOr(P.err, 1);
 }
 
-// How a launch of `tiles` row tiles in all, the longest of NG groups, runs
-// for B tokens on ncu CUs.
+// How a launch runs for B tokens on ncu CUs: `tiles` row tiles in all, which
+// make `wide` units of two tiles on eight wavefronts, the longest of NG groups.
 struct MmShape {
-  int CT, TM, KS, units, wgs;
+  int CT, TM, KS, NW, units, wgs;
 };
 
-static MmShape mm_shape(int64_t tiles, int NG, int32_t B, int ncu) {
+static MmShape mm_shape(int64_t tiles, int64_t wide, int NG, int32_t B, int ncu) {
   MmShape s{};
   s.CT = (B + 15) / 16;
   // Shared where its units (4 tiles a workgroup) still fill the CUs: 768
@@ -436,16 +446,35 @@ static MmShape mm_shape(int64_t tiles, int NG, int32_t B, int ncu) {
   // (one tile: 34.7), B = 16 31.9 (35.6), B = 64 47.2 (54.4); 768 tiles, B =
   // 8: 12.4 (10.0)
   s.TM = s.KS == 1 && tiles >= (int64_t)ncu * 4 ? 2 : 1;
+  // Eight wavefronts share the copies instead of four where that keeps the
+  // CUs busy.  One tile each, up to 8 tiles per CU, where four of two tiles
+  // leave one workgroup, four wavefronts, on a CU: 1536 tiles, B = 64 20.4 ->
+  // 18.6; 1250 tiles, K 12288: B = 8 26.7 -> 25.5, B = 64 44.7 -> 40.8.  Two
+  // tiles each beyond, which halves the copies per weight (3750 tiles: B = 64
+  // 35.1 -> 32.8; 96 FFN matrices: B = 16 430 -> 427, B = 32 475 -> 457, B =
+  // 64 587 -> 537; nothing to gain up to 8 tokens: 23.5 and 23.9), unless
+  // more than a tenth of the places for tiles stays empty in the rounds (10560
+  // tiles in 3 x 256 units of 16: B = 24 51.4 -> 55.6).
+  s.NW = kMWaves;
+  if (s.TM == 2) {
+    const int64_t places = (wide + ncu - 1) / ncu * ncu * (2 * kMWide);
+    if (tiles <= (int64_t)ncu * kMWide) {
+      s.NW = kMWide;
+      s.TM = 1;
+    } else if (B > 8 && tiles * 10 >= places * 9) {
+      s.NW = kMWide;
+    }
+  }
   return s;
 }
-static int mm_tiles_per_unit(const MmShape &s) { return s.TM * (kMWaves / s.KS); }
+static int mm_tiles_per_unit(const MmShape &s) { return s.TM * (s.NW / s.KS); }
 
-// Workgroups: all units at once up to two workgroups per CU.  A long pass
-// of up to 32 tokens runs one per CU: fewer streams read faster (96 FFN
-// matrices, B = 8: 463 us against 478, B = 32: 563 against 574; beyond 32
-// tokens the second workgroup's overlap is worth more: B = 64 694 against 679).
-static int mm_wgs(int units, int32_t B, int ncu) {
-  const int most = units >= 8 * ncu && B <= 32 ? ncu : 2 * ncu;
+// Workgroups: all units at once up to two workgroups per CU.  Eight
+// wavefronts are one workgroup per CU, and so is a long pass of up to 32
+// tokens: fewer streams read faster (96 FFN matrices, B = 8: 401 us against
+// 410; beyond 32 tokens the second workgroup's overlap is worth more).
+static int mm_wgs(int units, int NW, int32_t B, int ncu) {
+  const int most = NW > kMWaves || (units >= 8 * ncu && B <= 32) ? ncu : 2 * ncu;
   return units < most ? units : most;
 }
 
@@ -457,14 +486,16 @@ static int mm_ncu() {
 }
 
 static MmShape mm_setup(const MmJobSpec *jobs, int n, int32_t B, MmJob *out) {
-  int64_t tiles = 0;
+  int64_t tiles = 0, wide = 0;
   int NG = 0;
   for (int j = 0; j < n; ++j) {
-    tiles += (jobs[j].nrows + kTileRows - 1) / kTileRows;
+    const int64_t t = (jobs[j].nrows + kTileRows - 1) / kTileRows;
+    tiles += t;
+    wide += (t + 2 * kMWide - 1) / (2 * kMWide);
     NG = jobs[j].L.NG > NG ? jobs[j].L.NG : NG;
   }
   const int ncu = mm_ncu();
-  MmShape s = mm_shape(tiles, NG, B, ncu);
+  MmShape s = mm_shape(tiles, wide, NG, B, ncu);
   const int per = mm_tiles_per_unit(s);
   int unit = 0;
   for (int j = 0; j < n; ++j) {
@@ -484,13 +515,13 @@ static MmShape mm_setup(const MmJobSpec *jobs, int n, int32_t B, MmJob *out) {
     unit += (J.u.ntiles + per - 1) / per;
   }
   s.units = unit;
-  s.wgs = mm_wgs(unit, B, ncu);
+  s.wgs = mm_wgs(unit, s.NW, B, ncu);
   return s;
 }
 
-template <int TM, int CT, int KS, bool half8, bool plan>
+template <int NW, int TM, int CT, int KS, bool half8, bool plan>
 static hipError_t mm_launch1(const MmParams &P, int wgs, hipStream_t s) {
-  auto *const k = &matmul_kernel<TM, CT, KS, half8, plan>;
+  auto *const k = &matmul_kernel<NW, TM, CT, KS, half8, plan>;
   // dynamic LDS beyond the default limit: allowed once per process
   static const hipError_t attr = hipFuncSetAttribute(
       (const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
@@ -498,7 +529,7 @@ static hipError_t mm_launch1(const MmParams &P, int wgs, hipStream_t s) {
   constexpr size_t lds = mm_x_bytes(CT, KS, half8) +
                          (KS > 1 ? (size_t)2 * TM * CT * 4 * 64 * sizeof(int64_t) : 0);
   static_assert(lds <= kLdsBytes, "LDS of one workgroup");
-  hipLaunchKernelGGL(k, dim3(wgs), dim3(kMThreads), lds, s, P);
+  hipLaunchKernelGGL(k, dim3(wgs), dim3(64 * NW), lds, s, P);
   return hipGetLastError();
 }
 
@@ -506,11 +537,14 @@ template <int CT, bool plan>
 static hipError_t mm_launch2(const MmParams &P, const MmShape &c, hipStream_t s) {
   if constexpr (CT == 1) {
     // the split's private copies are halved for up to 8 tokens
-    if (c.KS > 1 && P.B <= 8) return mm_launch1<1, CT, kMWaves, true, plan>(P, c.wgs, s);
+    if (c.KS > 1 && P.B <= 8) return mm_launch1<kMWaves, 1, CT, kMWaves, true, plan>(P, c.wgs, s);
   }
-  if (c.KS > 1) return mm_launch1<1, CT, kMWaves, false, plan>(P, c.wgs, s);
-  return c.TM == 1 ? mm_launch1<1, CT, 1, false, plan>(P, c.wgs, s)
-                   : mm_launch1<2, CT, 1, false, plan>(P, c.wgs, s);
+  if (c.KS > 1) return mm_launch1<kMWaves, 1, CT, kMWaves, false, plan>(P, c.wgs, s);
+  if (c.NW > kMWaves)
+    return c.TM == 1 ? mm_launch1<kMWide, 1, CT, 1, false, plan>(P, c.wgs, s)
+                     : mm_launch1<kMWide, 2, CT, 1, false, plan>(P, c.wgs, s);
+  return c.TM == 1 ? mm_launch1<kMWaves, 1, CT, 1, false, plan>(P, c.wgs, s)
+                   : mm_launch1<kMWaves, 2, CT, 1, false, plan>(P, c.wgs, s);
 }
 
 template <bool plan>
@@ -549,7 +583,7 @@ hipError_t matmul_plan_prepare(const MmJobSpec *jobs, int n, int32_t B,
       u.ntiles -= t;
       u.row0 = t * kTileRows;
     }
-  *cfg = MmPlanCfg{B, s.CT, s.TM, s.KS, s.units, s.wgs};
+  *cfg = MmPlanCfg{B, s.CT, s.TM, s.KS, s.NW, s.units, s.wgs};
   return hipSuccess;
 }
 
@@ -561,7 +595,7 @@ hipError_t launch_matmul_plan(const void *d_table, const MmPlanCfg &cfg, int32_t
   P.B = cfg.B;
   P.err = err;
   P.tab = (const MmUnit *)d_table;
-  return mm_launch<true>(P, MmShape{cfg.CT, cfg.TM, cfg.KS, cfg.units, cfg.wgs}, s);
+  return mm_launch<true>(P, MmShape{cfg.CT, cfg.TM, cfg.KS, cfg.NW, cfg.units, cfg.wgs}, s);
 }
 
 hipError_t launch_matmul_multi(const MmJobSpec *jobs, int n, int32_t B, int32_t *err,
