@@ -221,8 +221,9 @@ struct HostIO {
   bool on;
   HostIO(w4a8_ctx *ctx, size_t in_bytes, size_t out_bytes) : c(ctx), on(false) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    on = c->h_pin && in_bytes <= kPinIn && out_bytes <= kPinOut &&
-         hipStreamIsCapturing(c->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+    if (!c->h_pin || in_bytes > kPinIn || out_bytes > kPinOut) return;
+    on = hipStreamIsCapturing(c->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+    if (!on) (void)hipGetLastError();   // the next launch reports its own
   }
   uint8_t *in() const { return c->h_pin + kPinCtl; }
   const uint8_t *out() const { return c->h_pin + kPinCtl + kPinIn; }
@@ -462,6 +463,7 @@ int w4a8_ctx_create(int32_t device, w4a8_ctx **out) {
         (void)hipHostFree(h);
       }
     }
+    if (!rc && !c->h_pin) (void)hipGetLastError();   // none: calls copy through HIP
   } while (0);
   if (rc) {
     w4a8_ctx_destroy(c);
