@@ -16,14 +16,14 @@
 // at or above the running entry[31] can insert or tie, and since entry[31]
 // only rises, an arrival below it when its 64-row group starts stays below.
 //
-// One wavefront per chunk.  A chunk publishes its own list; the last chunk
-// of each run of 16 (a super-chunk) also publishes the run's list.  The list
-// before chunk c is then the merge of at most 15 super lists and 15 chunk
-// lists.  A chunk only waits for lower-numbered chunks, each of which
-// publishes before it waits, so the waits end as long as every chunk's
-// wavefront runs; the last chunk gathers the result.  Flags carry an epoch,
-// so they are never cleared between uses; data crossing workgroups moves
-// with agent-coherent accesses.
+// In the plan, one wavefront per chunk (the kernel of its own has runs of four
+// chunks).  A chunk publishes its own list; the last chunk of each run of 16
+// (a super-chunk) also publishes the run's list.  The list before chunk c is
+// then the merge of at most 15 super lists and 15 chunk lists.  A chunk only
+// waits for lower-numbered chunks, each of which publishes before it waits,
+// so the waits end as long as every chunk's wavefront runs; the last chunk
+// gathers the result.  Flags carry an epoch, so they are never cleared
+// between uses; data crossing workgroups moves with agent-coherent accesses.
 #pragma once
 #include "w4a8_internal.h"
 
@@ -162,7 +162,7 @@ __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(0)" ::
 
 // Keys stream through buf (LDS, 128 keys) 64 lanes at a time: lanes with q
 // set append their key, and every full 64 are sorted and merged into L.
-// The wavefront is alone in its workgroup and its LDS accesses execute in
+// No other wavefront uses buf, and a wavefront's LDS accesses execute in
 // order, so only the compiler's ordering is fenced.
 struct TopFeed {
   uint64_t *buf;
@@ -253,21 +253,10 @@ __device__ __forceinline__ int64_t chunk_end(int c, int64_t n) {
   return n < e ? n : e;
 }
 
-// Chunk c's part of the scan, by one wavefront, from its values: yv[t] is
-// row chunk_first(c) + lane + 64 t (anything past the chunk's end).  rows
-// (kTkRows int32) and buf (128 keys) are this wavefront's LDS.  Flags
-// (epoch > 0): pub[c] = epoch once chunk c's list is in part[c]; spub[s] =
-// epoch once super-chunk s's list is in sup[s]; done[c] = 2 epoch + (chunk
-// c's replay set the overflow bit).  out = vals[32], rows[32], count,
-// overflow (entries past count are zero), written by the last chunk.
-// Returns false if a wait gave up after `spin` polls.
-__device__ bool chunk_run(const int32_t (&yv)[kTkPerLane], int32_t *rows, uint64_t *buf,
-                          int64_t n, int nchunks, int c, int32_t epoch, uint64_t *part,
-                          uint64_t *sup, int32_t *flags, int32_t *out, uint32_t spin, bool up,
-                          int lane) {
-  int32_t *pub = flags, *done = flags + kTopkMaxChunks, *spub = flags + 2 * kTopkMaxChunks;
-  const int64_t s0 = chunk_first(c);
-  const int64_t end = chunk_end(c, n);
+// A chunk's values (yv[t]: row s0 + lane + 64 t) into rows, and its top 32.
+__device__ __forceinline__ uint64_t chunk_top32(const int32_t (&yv)[kTkPerLane], int32_t *rows,
+                                                uint64_t *buf, int64_t s0, int64_t end, bool up,
+                                                int lane) {
   uint64_t keys[kTkPerLane];
 #pragma unroll
   for (int t = 0; t < kTkPerLane; ++t) {
@@ -275,25 +264,13 @@ __device__ bool chunk_run(const int32_t (&yv)[kTkPerLane], int32_t *rows, uint64
     rows[lane + 64 * t] = yv[t];
     keys[t] = r < end ? tk_key(yv[t], (uint32_t)r) : 0;
   }
-  const uint64_t own = top32_chunk(keys, buf, up, lane);
-  if (lane < kTk) st_coh64(part + (int64_t)c * kTk + lane, own);
-  wait_vm();
-  if (lane == 0) st_coh32(pub + c, epoch);
-  // the list of the earlier chunks of this super-chunk ...
-  const int s = c / kTopkSuper, c0 = s * kTopkSuper;
-  auto is_epoch = [epoch](int32_t v) { return v == epoch; };
-  bool ok = wait_words(pub + c0, c - c0, is_epoch, lane, spin);
-  const uint64_t W = top32_lists(part + (int64_t)c0 * kTk, c - c0, up, lane);
-  if (c - c0 == kTopkSuper - 1) {
-    const uint64_t S = merge32v(W, own, up, lane);   // all lanes take part in a merge
-    if (lane < kTk) st_coh64(sup + s * kTk + lane, S);
-    wait_vm();
-    if (lane == 0) st_coh32(spub + s, epoch);
-  }
-  // ... and of the earlier super-chunks: the list before this chunk
-  ok = wait_words(spub, s, is_epoch, lane, spin) && ok;
-  const uint64_t pre = merge32v(top32_lists(sup, s, up, lane), W, up, lane);
-  // replay this chunk's arrivals
+  return top32_chunk(keys, buf, up, lane);
+}
+
+// Replay a chunk's arrivals, rows [s0, end) with values rows[0..], against
+// the list before it; 1 where they set the overflow bit.
+__device__ __forceinline__ int chunk_replay(uint64_t pre, const int32_t *rows, int64_t s0,
+                                            int64_t end, bool up, int lane) {
   uint64_t L = pre;
   int32_t cv = tk_val(lane_u64(L, kTk - 1));   // entry 31's value (INT32_MIN while empty)
   int ovf = 0;
@@ -345,6 +322,43 @@ __device__ bool chunk_run(const int32_t (&yv)[kTkPerLane], int32_t *rows, uint64
       cv = pos < kTk - 1 ? e30 : (pos == kTk - 1 ? vj : cv);
     }
   }
+  return ovf;
+}
+
+// Chunk c's part of the scan, by one wavefront, from its values: yv[t] is
+// row chunk_first(c) + lane + 64 t (anything past the chunk's end).  rows
+// (kTkRows int32) and buf (128 keys) are this wavefront's LDS.  Flags
+// (epoch > 0): pub[c] = epoch once chunk c's list is in part[c]; spub[s] =
+// epoch once super-chunk s's list is in sup[s]; done[c] = 2 epoch + (chunk
+// c's replay set the overflow bit).  out = vals[32], rows[32], count,
+// overflow (entries past count are zero), written by the last chunk.
+// Returns false if a wait gave up after `spin` polls.
+__device__ bool chunk_run(const int32_t (&yv)[kTkPerLane], int32_t *rows, uint64_t *buf,
+                          int64_t n, int nchunks, int c, int32_t epoch, uint64_t *part,
+                          uint64_t *sup, int32_t *flags, int32_t *out, uint32_t spin, bool up,
+                          int lane) {
+  int32_t *pub = flags, *done = flags + kTopkMaxChunks, *spub = flags + 2 * kTopkMaxChunks;
+  const int64_t s0 = chunk_first(c);
+  const int64_t end = chunk_end(c, n);
+  const uint64_t own = chunk_top32(yv, rows, buf, s0, end, up, lane);
+  if (lane < kTk) st_coh64(part + (int64_t)c * kTk + lane, own);
+  wait_vm();
+  if (lane == 0) st_coh32(pub + c, epoch);
+  // the list of the earlier chunks of this super-chunk ...
+  const int s = c / kTopkSuper, c0 = s * kTopkSuper;
+  auto is_epoch = [epoch](int32_t v) { return v == epoch; };
+  bool ok = wait_words(pub + c0, c - c0, is_epoch, lane, spin);
+  const uint64_t W = top32_lists(part + (int64_t)c0 * kTk, c - c0, up, lane);
+  if (c - c0 == kTopkSuper - 1) {
+    const uint64_t S = merge32v(W, own, up, lane);   // all lanes take part in a merge
+    if (lane < kTk) st_coh64(sup + s * kTk + lane, S);
+    wait_vm();
+    if (lane == 0) st_coh32(spub + s, epoch);
+  }
+  // ... and of the earlier super-chunks: the list before this chunk
+  ok = wait_words(spub, s, is_epoch, lane, spin) && ok;
+  const uint64_t pre = merge32v(top32_lists(sup, s, up, lane), W, up, lane);
+  const int ovf = chunk_replay(pre, rows, s0, end, up, lane);
   if (c == nchunks - 1) {
     const uint64_t whole = merge32v(pre, own, up, lane);
     ok = wait_words(done, c, [epoch](int32_t v) { return (v >> 1) == epoch; }, lane, spin) && ok;
