@@ -212,7 +212,7 @@ int take_err(w4a8_ctx *c) {
 // into the staging buffer, and after the work one kernel writes the results
 // and the error word into the pinned block and raises a flag the host polls:
 // two launches instead of a driver copy per buffer and one for the error word
-// (matvec on 1000 x 1152: 70 -> 27 us a call).  Used where inputs and results
+// (matvec on 1000 x 1152: 70 -> 25 us a call).  Used where inputs and results
 // fit; never on a capturing stream (the flag would not rise).
 constexpr size_t kPinCtl = 256, kPinIn = 64 << 10, kPinOut = 160 << 10;
 
