@@ -236,9 +236,9 @@ struct HostIO {
     HIP_TRY(launch_host_copy(h, c->stream));
     return W4A8_OK;
   }
-  // n bytes at src (rounded up to 16) to out(), waited for; check: report
-  // (and clear) the error word
-  int receive(const void *src, size_t n, bool check) {
+  // n bytes at src (rounded up to 16) to out(), waited for; out() holds an
+  // earlier call's bytes where this fails
+  int receive(const void *src, size_t n) {
     volatile uint32_t *flag = (volatile uint32_t *)c->h_pin;
     HostCopy h{};
     h.src = src;
@@ -261,7 +261,11 @@ struct HostIO {
       }
     }
     std::atomic_thread_fence(std::memory_order_acquire);
-    if (!check || ((volatile int32_t *)c->h_pin)[1] == 0) return W4A8_OK;
+    return W4A8_OK;
+  }
+  // after receive: report (and clear) the error word that came with the results
+  int error() {
+    if (((volatile int32_t *)c->h_pin)[1] == 0) return W4A8_OK;
     HIP_TRY(hipStreamSynchronize(c->stream));
     return take_err(c);
   }
@@ -714,7 +718,7 @@ static int vec_prologue(w4a8_ctx *c, int32_t pro, const int16_t *x16,
     if ((rc = io.send(pro == PRO_RMSNORM_DYNQ8 ? 2 * nb : nb))) return rc;
     HIP_TRY(launch_vec_prologue(P, c->stream));
     // xn, x8 and e_x lie one after another
-    if ((rc = io.receive(d_xn, 2 * nb + 16, false))) return rc;
+    if ((rc = io.receive(d_xn, 2 * nb + 16))) return rc;
     if (xn) memcpy(xn, io.out(), nb);
     if (x8) memcpy(x8, io.out() + nb, n);
     if (e) memcpy(e, io.out() + 2 * nb, 4);
@@ -853,13 +857,13 @@ int w4a8_matvec_fused(w4a8_ctx *c, const w4a8_weights *w, int32_t prologue,
   if (rc) return rc;
   if (io.on) {
     // out, x8, e_x and the normalised vector lie one after another
-    rc = io.receive(d_out, out_b, true);
+    if ((rc = io.receive(d_out, out_b))) return rc;
     const uint8_t *h = io.out();
     memcpy(out, h, ob);
     if (x8_out) memcpy(x8_out, h + (o_x8 - o_out), K);
     if (e_x_io) memcpy(e_x_io, h + (o_e - o_out), 4);
     if (xn_out && rms) memcpy(xn_out, h + (o_xn - o_out), (size_t)K * 2);
-    return rc;
+    return io.error();
   }
   HIP_TRY(hipMemcpyAsync(out, d_out, ob, hipMemcpyDeviceToHost, c->stream));
   if (x8_out) HIP_TRY(hipMemcpyAsync(x8_out, s + o_x8, K, hipMemcpyDeviceToHost, c->stream));
