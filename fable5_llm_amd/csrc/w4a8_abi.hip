@@ -838,6 +838,16 @@ int w4a8_matvec_fused(w4a8_ctx *c, const w4a8_weights *w, int32_t prologue,
   if (rms && !norm_w) return fail(W4A8_E_ARG, "PRO_RMSNORM_DYNQ8 needs norm_w");
   const size_t in_b = rms ? o_w + (size_t)K * 2 : xb;
   const size_t out_b = (rms && xn_out ? o_xn + (size_t)K * 2 : o_e + 16) - o_out;
+  const int32_t ex_in = (prologue == PRO_X8 && e_x_io) ? *e_x_io : 0;
+  void *d_out = s + o_out;
+  // checked before anything is enqueued: a copy of the pinned block left on
+  // the stream by a refused call would read it while a later call, on another
+  // stream, fills it
+  GemvParams P;
+  rc = site_params(c, P, 1, &w, &epilogue, &p0, &d_out, prologue, s + o_x,
+                   (const int16_t *)(s + o_w), in_f, one_plus, ex_in, (int8_t *)(s + o_x8),
+                   (int32_t *)(s + o_e), (int16_t *)(s + o_xn));
+  if (rc) return rc;
   HostIO io(c, in_b, out_b);
   if (io.on) {
     memcpy(io.in(), x, xb);
@@ -848,13 +858,7 @@ int w4a8_matvec_fused(w4a8_ctx *c, const w4a8_weights *w, int32_t prologue,
     if (rms)
       HIP_TRY(hipMemcpyAsync(s + o_w, norm_w, (size_t)K * 2, hipMemcpyHostToDevice, c->stream));
   }
-  const int32_t ex_in = (prologue == PRO_X8 && e_x_io) ? *e_x_io : 0;
-  const int32_t ep = epilogue;
-  void *d_out = s + o_out;
-  rc = site_launch(c, 1, &w, &ep, &p0, &d_out, prologue, s + o_x,
-                   (const int16_t *)(s + o_w), in_f, one_plus, ex_in,
-                   (int8_t *)(s + o_x8), (int32_t *)(s + o_e), (int16_t *)(s + o_xn));
-  if (rc) return rc;
+  HIP_TRY(launch_gemv(P, grid_for(c, P.total_tiles), c->stream));
   if (io.on) {
     // out, x8, e_x and the normalised vector lie one after another
     if ((rc = io.receive(d_out, out_b))) return rc;

@@ -7,7 +7,7 @@ import sys
 import numpy as np
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-E_HIP, E_Y32_OVF = -5, -4
+E_HIP, E_Y32_OVF, E_RANGE = -5, -4, -7
 PRO_RMSNORM_DYNQ8, EPI_Y32 = 2, 0
 N_, K = 40, 256
 
@@ -55,5 +55,13 @@ def failed_copies():
     assert call()[:2] == (0, [True] * 4)
 
 
-{"failed_copies": failed_copies}[sys.argv[2]]()
+def refused_calls():
+    call()
+    before = rt.fake_launches()
+    rc, _, kept = call(in_f=41)
+    assert rc == E_RANGE and kept == [True] * 4
+    assert rt.fake_launches() == before, "a refused call left work on the stream"
+
+
+{"failed_copies": failed_copies, "refused_calls": refused_calls}[sys.argv[2]]()
 print("ok")

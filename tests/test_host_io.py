@@ -1,6 +1,7 @@
 """The host-buffer calls' host code on a stand-in for the HIP runtime
 (fake_hip.cpp; no GPU): a call whose results did not come back leaves the
-caller's buffers as they were."""
+caller's buffers as they were, and a call that is refused leaves nothing on
+the stream."""
 import os
 import subprocess
 import sys
@@ -22,7 +23,7 @@ def runtime(tmp_path_factory):
     return so
 
 
-@pytest.mark.parametrize("check", ["failed_copies"])
+@pytest.mark.parametrize("check", ["failed_copies", "refused_calls"])
 def test_host_calls(runtime, check):
     r = subprocess.run([sys.executable, os.path.join(HERE, "host_io_check.py"), runtime, check],
                        capture_output=True, text=True, timeout=120)
