@@ -26,9 +26,11 @@ def _dptr(t):
 
 
 def _i32s(values):
-    """int32 array of a sequence of whole numbers (OverflowError outside
-    int32)"""
-    return array("i", [int(v) for v in values])
+    """int32 array of a sequence of whole numbers, converted as numpy does"""
+    try:
+        return array("i", [*values])
+    except (TypeError, OverflowError):   # floats; arrays of wider types wrap
+        return array("i", np.ascontiguousarray(values, dtype=np.int32).tolist())
 
 
 def _aptr(a):

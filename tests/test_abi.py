@@ -73,3 +73,17 @@ def test_device_wrappers_refuse_short_buffers():
     E._dev(None, 4, "x", required=False)
     with pytest.raises(ValueError, match="device tensor"):
         E._dev(torch.zeros(4, dtype=torch.int32), 16, "x")
+
+
+def test_int_arguments_as_numpy_took_them():
+    # epilogues and p0s: what np.ascontiguousarray(..., dtype=np.int32) takes
+    # (arrays of other whole-number types wrap), and what it refuses
+    import numpy as np
+    from fable5_llm_amd import engine as E
+    for v in ([1, -2], (3,), np.array([5, -6]), np.array([0xFFFFFFFE, 7], dtype=np.uint32),
+              np.array([(1 << 32) + 9], dtype=np.int64), np.arange(6, dtype=np.int16)[::2],
+              [np.uint32(12)], [True, 2], [1.0, -2.0], np.array([3.0])):
+        assert list(E._i32s(v)) == np.ascontiguousarray(v, dtype=np.int32).tolist(), v
+    for v in ([1 << 31], [-(1 << 31) - 1]):
+        with pytest.raises(OverflowError):
+            E._i32s(v)
