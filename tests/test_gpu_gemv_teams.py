@@ -79,3 +79,31 @@ def test_prologue_extremes(engine, fill, K):
                 assert np.array_equal(x8, wx8) and e == we
     finally:
         w.free()
+
+
+@pytest.mark.parametrize("K", [128, 1152, 2176, 4096])   # 1, 2, 3 and 4 blocks a tile
+def test_argmax_in_step(engine, K):
+    # a long head: the winner, and a tie after it, in a tile that each of a
+    # team's four wavefronts finishes, those without blocks of it too
+    G = engine.grid
+    rows = (9 * G + 200) * 16 - 7            # four tile iterations for team 0
+    rng = np.random.default_rng(K)
+    img, _ = rand_image(rng, rows, K)
+    x16 = activation_x16(rng, K)
+    x8, _ = law.dyn_quant_i8(x16)
+    sh = law.sh_for_k(K)
+    best, _ = law.pack_ddr_rows(np.where(x8 >= 0, 7, -8).astype(np.int8)[None],
+                                np.full((1, K // 128), 65535, np.uint16))
+    best = np.frombuffer(best, np.uint8) if isinstance(best, bytes) else np.asarray(best).reshape(-1)
+    for it in range(4):
+        im = img.reshape(rows, -1).copy()
+        win = (3 * G * it + 5) * 16 + 3      # tile 5 of team 0's iteration
+        im[win] = best
+        im[win + 16] = best                  # the next workgroup's tile
+        w = engine.upload(im.reshape(-1), rows, K, sh)
+        try:
+            want = law.amax32(cfast.matvec_y32_img(im.reshape(-1), rows, K, sh, x8))
+            assert want[0] == win
+            assert tuple(engine.head_argmax(w, x16, prologue=N.PRO_DYNQ8)) == tuple(want), it
+        finally:
+            w.free()
