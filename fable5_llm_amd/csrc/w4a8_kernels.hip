@@ -444,12 +444,16 @@ constexpr int kGTeams = kGWaves / 4;
 constexpr int kPW0 = 4;                // teams 1 and 2 (wavefronts 4..11) run the prologue
 constexpr int kPT = kGT - 64 * kPW0;   // 512 threads
 
-// The LDS slots in which a team's tiles meet: tile `it` in slot it % kSlots.
-constexpr int kSlots = 8;
+// The LDS slots in which a team's tiles meet, where it has no more than two
+// (a longer stream goes in step, below): tile iteration `it` in slot it, used
+// once, so nothing is cleared for reuse or waited for.  Zeroed before the
+// workgroup meets, so their number is on the launch's path (eight a team:
+// 4096 x 4096 5.26 us in a graph of launches, two: 5.10).
+constexpr int kSlots = 2;
 struct TileSlot {
-  uint64_t sum[kTileRows];   // 16 * p of each row, zero between tiles
+  uint64_t sum[kTileRows];   // 16 * p of each row
   int32_t cnt;               // wavefronts that have added
-  int32_t gen;               // tiles the slot has finished
+  int32_t pad;
 };
 __device__ __forceinline__ void lds_add_u64(uint64_t *p, uint64_t v) {
   asm volatile("ds_add_u64 %0, %1" :: "v"(lds_off(p)), "v"(v) : "memory");
@@ -467,27 +471,16 @@ __device__ __forceinline__ int64_t quarter_sum(int64_t p) {
   return (int64_t)((uint64_t)p + dpp_u64<0x4E, 0xF>((uint64_t)p));
 }
 
-// Add this wavefront's share of a tile (quarter_sum) to the tile's slot; true in the wavefront that adds last of nw, which gets lane
-// l < 16's row sum in tot and leaves the slot free.  (A wavefront's LDS
-// instructions execute in order, so the count follows the sums.)
-__device__ __forceinline__ bool tile_add(TileSlot *slots, int it, int nw, int64_t p, int lane,
-                                         bool &ok, int64_t &tot) {
-  TileSlot &S = slots[it % kSlots];
-  // the tile that had the slot before is done (a wavefront is rarely 8 tiles
-  // ahead of its team)
-  if (it >= kSlots) ok = lds_wait_ge(&S.gen, it / kSlots) && ok;
+// Add this wavefront's share of a tile (quarter_sum) to the tile's slot; true
+// in the wavefront that adds last of nw, which gets lane l < 16's row sum in
+// tot.  (A wavefront's LDS instructions execute in order, so the count
+// follows the sums.)
+__device__ __forceinline__ bool tile_add(TileSlot &S, int nw, int64_t p, int lane, int64_t &tot) {
   if ((lane & 3) == 0) lds_add_u64(&S.sum[lane >> 2], (uint64_t)p);
   int32_t old = 0;
   if (lane == 0) old = lds_add_rtn(&S.cnt, 1);
   if (__builtin_amdgcn_readfirstlane(old) != nw - 1) return false;
-  if (lane < kTileRows) {
-    tot = (int64_t)lds_read_u64(&S.sum[lane]);
-    lds_post_u64(&S.sum[lane], 0);
-  }
-  if (lane == 0) {
-    lds_post_i32(&S.cnt, 0);
-    lds_post_i32(&S.gen, it / kSlots + 1);
-  }
+  if (lane < kTileRows) tot = (int64_t)lds_read_u64(&S.sum[lane]);
   return true;
 }
 
@@ -562,7 +555,7 @@ __global__ __launch_bounds__(kGT) void gemv_kernel(GemvParams P) {
   // without).  Short launches (up to two tiles per team) run without: no team
   // waits for another's first blocks (chained step in graph mode 1.33 ms in
   // step from the second tile on, 1.29 ms without).
-  const bool lockstep = T > 2 * VS;
+  const bool lockstep = T > kSlots * VS;
   if (lockstep)
     for (int i = tid; i < (int)(sizeof(red) / 4); i += kGT) ((int32_t *)red)[i] = 0;
 
@@ -638,7 +631,7 @@ __global__ __launch_bounds__(kGT) void gemv_kernel(GemvParams P) {
   // blocks of a tile (K <= 3072) too.  Left to the wavefronts that have
   // blocks, the epilogues are all one wavefront's where a tile is one block
   // (K <= 1024): 248,320 x 1024 with argmax 53.5 us, 43.9 in turn; 64,000 x
-  // 640 with MOVY int16 15.3 and 13.0; nothing changes from K = 4096 on.
+  // 640 with MOVY int16 15.4 and 13.1; nothing changes from K = 4096 on.
   int fin = 0;   // tile iterations finished
   auto finish_in_step = [&](int tg, int lane) {
     const int par = fin & 1;
@@ -667,7 +660,7 @@ __global__ __launch_bounds__(kGT) void gemv_kernel(GemvParams P) {
         finish_in_step(tg, lane);
       } else {
         int64_t tot = 0;
-        if (tile_add(slots[team], it, nw, p, lane, grp.ok, tot)) finish(tg, tot, lane);
+        if (tile_add(slots[team][it], nw, p, lane, tot)) finish(tg, tot, lane);
       }
       p = 0;
     }

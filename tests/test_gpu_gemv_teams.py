@@ -26,6 +26,7 @@ def _expect(img, n, K, sh, pro, x, nw):
     (4096, 4096), (4097, 4096), (4113, 1024),     # 256 tiles, one more, two more
     (33, 4224), (4096, 12288), (4096, 8192), (4100, 8192), (300, 5248),   # one team of twelve
     (8200, 2048), (12289, 4096), (12304, 8192),   # two and three tiles a workgroup
+    (24576, 1024), (24570, 4224), (24576, 128),   # two a team
     (24592, 1024), (24592, 4224), (24590, 128),   # two a team and one more: in step from here
     (40000, 512), (37000, 3200),
 ])
