@@ -424,45 +424,55 @@ __global__ __launch_bounds__(64 * NW, 2) void matmul_kernel(MmParams P) {
   if (ovf) atomicOr(P.err, 1);
 }
 
-// How a launch runs for B tokens on ncu CUs: `tiles` row tiles in all, which
-// make `wide` units of two tiles on eight wavefronts, the longest of NG groups.
+// How a launch runs for B tokens on ncu CUs.
 struct MmShape {
   int CT, TM, KS, NW, units, wgs;
 };
 
-static MmShape mm_shape(int64_t tiles, int64_t wide, int NG, int32_t B, int ncu) {
+// `tiles` row tiles of `groups` groups in all, the longest of NG, which make
+// `quads` units of four tiles and `wide` units of sixteen.
+static MmShape mm_shape(int64_t tiles, int64_t groups, int64_t quads, int64_t wide, int NG,
+                        int32_t B, int ncu) {
   MmShape s{};
   s.CT = (B + 15) / 16;
   // Shared where its units (4 tiles a workgroup) still fill the CUs: 768
   // tiles (3 per CU) at B = 8, 10.0 us shared, 9.8 split; 512 tiles, 9.7 and
-  // 7.5; 1536 tiles, 14.0 and 14.4.  Beyond 32 tokens the shared copies are
-  // worth more (512 tiles, B = 48: 13.1 and 15.4; 384 tiles, K 8192: 21.0 and
-  // 21.5), and up to K = 2048 the split leaves wavefronts without groups (625
-  // tiles, K 1024, B = 24: 6.5 and 8.5).
-  const int64_t need = B > 32 || NG <= 16 ? ncu * 3 / 2 : ncu * 3;
+  // 7.5.  Beyond 32 tokens the shared copies are worth more (512 tiles, B =
+  // 48: 13.1 and 15.4; 384 tiles, K 8192: 21.0 and 21.5), and up to K = 2048
+  // the split leaves wavefronts without groups (625 tiles, K 1024, B = 24: 6.5
+  // and 8.5).  Tiles of 48 groups and more (K = 6144): few tokens stay split
+  // for longer, their copies being small beside the weights (768 tiles, K 12288:
+  // B = 8 24.5 shared, 18.7 split, B = 16 24.8 and 23.5; 960 tiles, B = 8 23.8
+  // and 23.3, B = 16 23.9 and 29.0), 17 to 32 go shared once the split's two
+  // workgroups per CU are full (640 tiles, K 12288, B = 24 25.6 and 26.8; 512
+  // tiles 23.5 and 20.5).
+  int64_t need = B > 32 || NG <= 16 ? ncu * 3 / 2 : ncu * 3;
+  if (groups >= 48 * tiles) {
+    if (B <= 8) need = ncu * 4;
+    else if (B <= 16) need = ncu * 3 + 1;
+    else if (B <= 32) need = ncu * 2 + 1;
+  }
   s.KS = tiles >= need ? 1 : kMWaves;
-  // two tiles a wavefront share its reads of the activations, once that
-  // leaves a workgroup for every other CU: 1250 tiles, K 12288: B = 8 35.4
-  // (one tile: 34.7), B = 16 31.9 (35.6), B = 64 47.2 (54.4); 768 tiles, B =
-  // 8: 12.4 (10.0)
-  s.TM = s.KS == 1 && tiles >= (int64_t)ncu * 4 ? 2 : 1;
-  // Eight wavefronts share the copies instead of four where that keeps the
-  // CUs busy.  One tile each, up to 8 tiles per CU, where four of two tiles
-  // leave one workgroup, four wavefronts, on a CU: 1536 tiles, B = 64 20.4 ->
-  // 18.6; 1250 tiles, K 12288: B = 8 26.7 -> 25.5, B = 64 44.7 -> 40.8.  Two
-  // tiles each beyond, which halves the copies per weight (3750 tiles: B = 64
-  // 35.1 -> 32.8; 96 FFN matrices: B = 16 430 -> 427, B = 32 475 -> 457, B =
-  // 64 587 -> 537; nothing to gain up to 8 tokens: 23.5 and 23.9), unless
-  // more than a tenth of the places for tiles stays empty in the rounds (10560
-  // tiles in 3 x 256 units of 16: B = 24 51.4 -> 55.6).
+  s.TM = 1;
   s.NW = kMWaves;
-  if (s.TM == 2) {
-    const int64_t places = (wide + ncu - 1) / ncu * ncu * (2 * kMWide);
-    if (tiles <= (int64_t)ncu * kMWide) {
-      s.NW = kMWide;
-      s.TM = 1;
-    } else if (B > 8 && tiles * 10 >= places * 9) {
-      s.NW = kMWide;
+  // Beyond one unit of four tiles per CU eight wavefronts share the copies,
+  // one tile each, which keeps a workgroup on every CU busy where four
+  // would leave most CUs with one (1280 tiles, K 4096, B = 8 / 64: 12.4 / 19.0
+  // on eight, 12.6 / 21.5 on four, K 12288, B = 64 45.2 and 53.8; up to one
+  // per CU four are better: 1024 tiles, K 4096 12.0 / 18.0 and 10.7 / 15.8, K
+  // 12288, B = 8 28.7 and 23.7).
+  if (s.KS == 1 && tiles >= ncu * 4 && quads > ncu) {
+    s.NW = kMWide;
+    // Beyond 8 tiles per CU two tiles a wavefront share its reads of the
+    // activations, on eight wavefronts (3750 tiles: B = 64 35.1 on four, 32.8;
+    // 96 FFN matrices: B = 32 475 and 457, B = 64 587 and 537), except up to
+    // 8 tokens (23.5 and 23.9) and where more than a tenth of the places for
+    // tiles stays empty in the rounds (10560 tiles in 3 x 256 units of 16: B =
+    // 24 51.4 and 55.6).
+    if (tiles > (int64_t)ncu * kMWide) {
+      s.TM = 2;
+      const int64_t places = (wide + ncu - 1) / ncu * ncu * (2 * kMWide);
+      if (B <= 8 || tiles * 10 < places * 9) s.NW = kMWaves;
     }
   }
   return s;
@@ -486,16 +496,18 @@ static int mm_ncu() {
 }
 
 static MmShape mm_setup(const MmJobSpec *jobs, int n, int32_t B, MmJob *out) {
-  int64_t tiles = 0, wide = 0;
+  int64_t tiles = 0, groups = 0, quads = 0, wide = 0;
   int NG = 0;
   for (int j = 0; j < n; ++j) {
     const int64_t t = (jobs[j].nrows + kTileRows - 1) / kTileRows;
     tiles += t;
+    groups += t * jobs[j].L.NG;
+    quads += (t + kMWaves - 1) / kMWaves;
     wide += (t + 2 * kMWide - 1) / (2 * kMWide);
     NG = jobs[j].L.NG > NG ? jobs[j].L.NG : NG;
   }
   const int ncu = mm_ncu();
-  MmShape s = mm_shape(tiles, wide, NG, B, ncu);
+  MmShape s = mm_shape(tiles, groups, quads, wide, NG, B, ncu);
   const int per = mm_tiles_per_unit(s);
   int unit = 0;
   for (int j = 0; j < n; ++j) {

@@ -1,7 +1,7 @@
 // A stand-in for the HIP runtime on a machine without a GPU, for tests of the
-// library's host code: device memory is host memory filled with 0x11, kernels
-// do nothing except host_copy_kernel, whose copies are made, and one launch,
-// wait or flag can be made to fail.  Built as libamdhip64.so.7 and loaded
+// library's host code: device memory is host memory, its first MiB filled with
+// 0x11, kernels do nothing except host_copy_kernel, whose copies are made, and
+// one launch, wait or flag can be made to fail.  Built as libamdhip64.so.7 and loaded
 // before the library, in a process of its own.
 #include <map>
 #include <string>
@@ -13,6 +13,8 @@
 
 namespace {
 std::map<const void *, std::string> names;
+std::string last_name;
+unsigned last_grid;
 int launches, fail_in, sync_fails, flag_lost, device_error;
 struct Config {
   dim3 grid, block;
@@ -20,8 +22,10 @@ struct Config {
   hipStream_t stream;
 } config;
 
-hipError_t launch(const void *f, void **args) {
+hipError_t launch(const void *f, dim3 grid, void **args) {
   ++launches;
+  last_name = names[f];
+  last_grid = grid.x;
   if (fail_in > 0 && --fail_in == 0) return hipErrorLaunchFailure;
   if (names[f].find("host_copy_kernel") != std::string::npos) {
     const w4a8::HostCopy &c = *(const w4a8::HostCopy *)args[0];
@@ -43,8 +47,9 @@ hipError_t note(hipError_t e) {
 
 extern "C" {
 
-// what the test sets and reads: the launch that fails (1: the next), whether
-// waits fail, whether copies' flags stay down, the error word kernels leave
+// what the tests set and read: the launch that fails (1: the next), whether
+// waits fail, whether copies' flags stay down, the error word kernels leave;
+// the launches so far, and the last one's kernel and grid
 void fake_set(int fail, int sync, int lost, int err) {
   fail_in = fail;
   sync_fails = sync;
@@ -52,6 +57,10 @@ void fake_set(int fail, int sync, int lost, int err) {
   device_error = err;
 }
 int fake_launches(void) { return launches; }
+const char *fake_last_kernel(unsigned *grid) {
+  *grid = last_grid;
+  return last_name.c_str();
+}
 
 void **__hipRegisterFatBinary(const void *) {
   static void *module;
@@ -74,16 +83,16 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *n, hipStream_t *s
   *s = config.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t) {
-  return note(launch(f, args));
+hipError_t hipLaunchKernel(const void *f, dim3 g, dim3, void **args, size_t, hipStream_t) {
+  return note(launch(f, g, args));
 }
-hipError_t hipExtLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t,
+hipError_t hipExtLaunchKernel(const void *f, dim3 g, dim3, void **args, size_t, hipStream_t,
                               hipEvent_t, hipEvent_t, int) {
-  return note(launch(f, args));
+  return note(launch(f, g, args));
 }
-hipError_t hipLaunchCooperativeKernel(const void *f, dim3, dim3, void **args, unsigned,
+hipError_t hipLaunchCooperativeKernel(const void *f, dim3 g, dim3, void **args, unsigned,
                                       hipStream_t) {
-  return note(launch(f, args));
+  return note(launch(f, g, args));
 }
 hipError_t hipGetLastError(void) {
   const hipError_t e = last;
@@ -94,7 +103,7 @@ const char *hipGetErrorString(hipError_t) { return "an error"; }
 
 static hipError_t allocate(void **p, size_t n) {
   *p = aligned_alloc(4096, (n + 4095) / 4096 * 4096);
-  memset(*p, 0x11, n);
+  memset(*p, 0x11, n < (1 << 20) ? n : 1 << 20);
   return hipSuccess;
 }
 hipError_t hipMalloc(void **p, size_t n) { return allocate(p, n); }

@@ -1,18 +1,17 @@
 """Run by test_host_io.py in a process of its own, with the stand-in runtime
 loaded before the library: host_io_check.py RUNTIME CHECK."""
 import ctypes
-import os
 import sys
 
 import numpy as np
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+import fake_hip
+
 E_HIP, E_Y32_OVF, E_RANGE = -5, -4, -7
 PRO_RMSNORM_DYNQ8, EPI_Y32 = 2, 0
 N_, K = 40, 256
 
-rt = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-lib = ctypes.CDLL(os.path.join(ROOT, "fable5_llm_amd", "libfable5_w4a8.so"))
+rt, lib = fake_hip.load(sys.argv[1])
 P = ctypes.c_void_p
 ctx, w = P(), P()
 assert lib.w4a8_ctx_create(0, ctypes.byref(ctx)) == 0
