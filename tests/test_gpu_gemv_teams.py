@@ -24,8 +24,9 @@ def _expect(img, n, K, sh, pro, x, nw):
 @pytest.mark.parametrize("rows,K", [
     (16, 128), (100, 640), (272, 1024),           # one block or none per wavefront
     (4096, 4096), (4097, 4096), (4113, 1024),     # 256 tiles, one more, two more
-    (33, 4224), (4096, 12288), (4096, 8192), (4100, 8192), (300, 5248),   # one team of twelve
-    (8200, 2048), (12289, 4096), (12304, 8192),   # two and three tiles a workgroup
+    (33, 4224), (4096, 12288), (4096, 8192), (300, 5248),   # one team of twelve
+    (4100, 8192),                                 # ... and a tile too many for it
+    (8200, 2048), (12289, 4096), (12304, 8192),   # up to three and four tiles a workgroup
     (24576, 1024), (24570, 4224), (24576, 128),   # two a team
     (24592, 1024), (24592, 4224), (24590, 128),   # two a team and one more: in step from here
     (40000, 512), (37000, 3200),

@@ -1,8 +1,8 @@
 """The batched kernel's units of eight wavefronts at their edges: one tile each
-(up to 8 tiles per CU) and two (beyond, where the rounds are nearly full), with
-every count of token tiles, quads of groups that end early, ragged rows and
-last units of one tile; and the four-wavefront units on the other side of each
-line.  Whole numbers, compared bit for bit with the C oracle per token."""
+(beyond a unit of four tiles per CU, up to 8 tiles per CU) and two (beyond,
+where the rounds are nearly full), with every count of token tiles, quads of
+groups that end early, ragged rows and last units of one tile; and the
+four-wavefront units on the other side of each line.  Whole numbers, compared bit for bit with the C oracle per token."""
 import numpy as np
 import pytest
 
@@ -14,17 +14,21 @@ pytestmark = pytest.mark.gpu
 GUARD = 0x5A5A5A5A
 
 
+# The forms on 256 CUs, as in test_gpu_matmul_units.py
+CASES = {
+    # four wavefronts of one tile: 1024 tiles, a unit on every CU
+    (4, 1, 1): [([16369], 128, 1)],
+    # eight of one tile: up to 2048 tiles
+    (8, 1, 1): [([16400, 20], 1152, 9), ([16600], 640, 33), ([32768], 256, 64)],
+    # four of two tiles: past 2048 tiles, rounds not full; and up to 8 tokens
+    (4, 2, 1): [([32770], 128, 17), ([60001], 128, 8)],
+    # eight of two tiles: 233 to 253 units on as many workgroups, 510 on 256
+    (8, 2, 1): [([60001], 128, 9), ([64497, 5], 384, 17), ([59500], 640, 48), ([130400], 128, 64)],
+}
+
+
 @pytest.mark.parametrize("plan", [False, True])
-@pytest.mark.parametrize("rows,K,B", [
-    # one tile a wavefront: 1024 to 2048 tiles on 256 CUs
-    ([16369], 128, 1), ([16400, 20], 1152, 9), ([16600], 640, 33), ([32768], 256, 64),
-    # four wavefronts of two tiles: past 2048 tiles, rounds not full
-    ([32770], 128, 17),
-    # two tiles a wavefront: 233 to 253 units on as many workgroups, 510 on 256
-    ([60001], 128, 9), ([64497, 5], 384, 17), ([59500], 640, 48), ([130400], 128, 64),
-    # ... and four wavefronts up to 8 tokens
-    ([60001], 128, 8),
-])
+@pytest.mark.parametrize("rows,K,B", sum(CASES.values(), []))
 def test_matmul_wide_units(engine, rows, K, B, plan):
     import torch
 

@@ -398,10 +398,10 @@ def test_matmul_plan_one_launch(engine, B):
     path holds; shapes from 40 x 256 to 4096 x 12288, several sharing x8)
     in one launch: every output equal to the per-launch path's (itself
     checked per token above) and the oracle's on three tokens; a second run
-    on overwritten outputs and graph replays give the same.  Up to 32 tokens
-    the 4096- and 4000-row matrices (and at 17..32 the 2048-row one) run
-    split into K slices whose sums meet across workgroups, so the reruns and
-    replays also check that a run leaves its reduction buffers zero."""
+    on overwritten outputs and graph replays give the same.  The 6,900
+    tiles run as units of two tiles on four wavefronts, several units to a
+    workgroup, from K = 12288 down to 128; the other forms' plans are in
+    test_gpu_matmul_units.py and test_gpu_matmul_wide.py."""
     import torch
     from fable5_llm_amd.engine import MatmulPlan
     rng = np.random.default_rng(4100 + B)

@@ -5,6 +5,8 @@ import json
 import pytest
 
 import fake_hip
+import test_gpu_matmul_units as units
+import test_gpu_matmul_wide as wide
 
 SPLIT, SHARED, WIDE, TWO, WIDE_TWO = (4, 1, 4), (4, 1, 1), (8, 1, 1), (4, 2, 1), (8, 2, 1)
 
@@ -46,3 +48,23 @@ def test_lines_of_the_rule(runtime):
     assert forms(runtime, [([16 * 1019, 32, 48], 128, 16, False)])[0] == ((8, 1, 1, 1, 0, 0), 130)
     assert forms(runtime, [([16 * 700, 16 * 100], [1024, 12288], 8, True)])[0][0] == \
         (4, 1, 1, 1, 0, 1)
+
+
+def test_gpu_cases_cover_every_instance(runtime):
+    # the GPU tests' cases take the form they are listed under, and together
+    # every instance that a launch can take
+    listed = [(form, list(c)) for m in (units, wide) for form, cs in m.CASES.items() for c in cs]
+    listed += [(SPLIT, list(c)) for c in units.MIXED]
+    got = forms(runtime, [c + [plan] for _, c in listed for plan in (False, True)])
+    seen = set()
+    for i, (f, grid) in enumerate(got):
+        form, (rows, K, B) = listed[i // 2]
+        assert (f[0], f[1], f[3]) == form, (rows, K, B)
+        if (rows, K, B) in units.MIXED:      # ... and a workgroup has several units
+            assert sum(-(-n // 16) for n in rows) > grid
+        seen.add(f)
+    every = {(4, 1, ct, 4, h, p) for ct in (1, 2, 3, 4) for h in ((0, 1) if ct == 1 else (0,))
+             for p in (0, 1)}
+    every |= {(nw, tm, ct, 1, 0, p) for nw in (4, 8) for tm in (1, 2) for ct in (1, 2, 3, 4)
+              for p in (0, 1)}
+    assert seen == every, (every - seen, seen - every)
