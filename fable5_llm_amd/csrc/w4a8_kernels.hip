@@ -26,8 +26,8 @@ namespace w4a8 {
 // instruction (v_pk_*_i16), wide products are 32 x 32 + 64 multiply-adds on
 // magnitudes, and a reduction is one LDS round trip (GroupRed).  From the
 // first workgroup's start to the first dot product, K = 4096: DYNQ8 3.3 ->
-// 2.4 us, RMSNorm 5.6 -> 3.9 us; a layer's FFN block 25.3 -> 23.4 us, the
-// chained step in graph mode 1.405 -> 1.306 ms.
+// 2.4 us, RMSNorm 5.6 -> 3.9 us; with the way tiles meet (below) a layer's FFN
+// block 25.4 -> 23.2 us, the chained step in graph mode 1.404 -> 1.291 ms.
 // ---------------------------------------------------------------------------
 typedef short s16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));

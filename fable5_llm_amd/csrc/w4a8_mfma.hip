@@ -34,15 +34,17 @@
 // wavefront) and the copies run on across them, so the stream does not drain
 // between tiles or matrices.  No wait depends on another workgroup.
 //
-// Measured, cold weights, us per launch: with a scale load per group and four
-// wavefronts everywhere -> now (a pass took 534, 711 and 4040 us with one
-// workgroup per CU, loader wavefronts and 8 slots):
-//   12288 + 12288 rows, K 4096:  B = 8: 13.7 -> 13.3, B = 64: 21.1 -> 18.6
-//   4096 rows, K 12288:          B = 8: 8.8 -> 8.6, B = 64: 19.2 -> 18.4
-//   60,000 rows, K 4096:         B = 8: 25.7 -> 23.9, B = 32: 29.4 -> 26.0, B = 64: 36.7 -> 32.8
-//   a pass of 96 FFN matrices:   B = 8: 430 -> 402, B = 32: 531 -> 457, B = 64: 625 -> 537
-// The pass's weights alone take 360 us at the read ceiling; the 117 MB of y32
-// that it writes at B = 32 take about 50 us of the rest.
+// Measured in a graph of launches, us each, weights cold in all of them, with
+// one workgroup per CU, loader wavefronts and 8 slots -> now:
+//   12288 + 12288 rows, K 4096:  B = 8: 18.9 -> 12.9, B = 64: 100 -> 19.4
+//   4096 rows, K 12288:          B = 8: 12.9 -> 9.4, B = 64: 52.5 -> 18.5
+//   60,000 rows, K 4096:         B = 8: 32.7 -> 25.4, B = 32: 51.4 -> 27.6, B = 64: 240 -> 35.8
+//   a pass of 96 FFN matrices:   B = 8: 525 -> 400, B = 32: 695 -> 450, B = 64: 4052 -> 539
+//   ... three passes' plans in turn:    538 -> 415,         708 -> 498,         4052 -> 568
+// Repeated, a pass finds part of its y32 (117 MB at B = 32) still in the
+// last-level cache; in turn, it does not.  Likewise three sets of 12288 +
+// 12288 rows in turn (156 MB) partly stay there: B = 8 11.9.  The pass's
+// weights alone take 360 us at the read ceiling.
 #include <algorithm>
 
 #include "w4a8_device.h"
@@ -435,17 +437,18 @@ static MmShape mm_shape(int64_t tiles, int64_t groups, int64_t quads, int64_t wi
                         int32_t B, int ncu) {
   MmShape s{};
   s.CT = (B + 15) / 16;
-  // Shared where its units (4 tiles a workgroup) still fill the CUs: 768
-  // tiles (3 per CU) at B = 8, 10.0 us shared, 9.8 split; 512 tiles, 9.7 and
-  // 7.5.  Beyond 32 tokens the shared copies are worth more (512 tiles, B =
-  // 48: 13.1 and 15.4; 384 tiles, K 8192: 21.0 and 21.5), and up to K = 2048
-  // the split leaves wavefronts without groups (625 tiles, K 1024, B = 24: 6.5
-  // and 8.5).  Tiles of 48 groups and more (K = 6144): few tokens stay split
-  // for longer, their copies being small beside the weights (768 tiles, K 12288:
-  // B = 8 24.5 shared, 18.7 split, B = 16 24.8 and 23.5; 960 tiles, B = 8 23.8
-  // and 23.3, B = 16 23.9 and 29.0), 17 to 32 go shared once the split's two
-  // workgroups per CU are full (640 tiles, K 12288, B = 24 25.6 and 26.8; 512
-  // tiles 23.5 and 20.5).
+  // Shared where its units (4 tiles a workgroup) still fill the CUs (K 4096,
+  // B = 8: 768 tiles, 3 per CU, 9.8 us shared, 9.3 split; 832 9.8 and 10.0;
+  // 512 9.2 and 7.1).  Beyond 32 tokens the shared copies are worth more (K
+  // 4096, B = 48: 384 tiles 12.7 and 13.3, 512 12.8 and 14.0), and up to K =
+  // 2048 the split leaves wavefronts without groups (B = 24: 640 tiles, K 1024
+  // 6.2 and 7.7, K 2048 7.9 and 8.2; 384 tiles, K 1024 5.7 and 6.5, but K 2048,
+  // B = 8 6.0 and 5.1).  Tiles of 48 groups and more (K = 6144): few tokens
+  // stay split for longer, their copies being small beside the weights (K
+  // 12288: 768 tiles, B = 8 24.5 and 18.7, B = 16 24.8 and 23.5; 960 tiles, B
+  // = 8 23.8 and 23.3, B = 16 23.9 and 29.0), 17 to 32 go shared once the
+  // split's two workgroups per CU are full (K 12288, B = 24: 640 tiles 25.6
+  // and 26.8, 512 23.5 and 20.5).
   int64_t need = B > 32 || NG <= 16 ? ncu * 3 / 2 : ncu * 3;
   if (groups >= 48 * tiles) {
     if (B <= 8) need = ncu * 4;
@@ -464,11 +467,14 @@ static MmShape mm_shape(int64_t tiles, int64_t groups, int64_t quads, int64_t wi
   if (s.KS == 1 && tiles >= ncu * 4 && quads > ncu) {
     s.NW = kMWide;
     // Beyond 8 tiles per CU two tiles a wavefront share its reads of the
-    // activations, on eight wavefronts (3750 tiles: B = 64 35.1 on four, 32.8;
-    // 96 FFN matrices: B = 32 475 and 457, B = 64 587 and 537), except up to
-    // 8 tokens (23.5 and 23.9) and where more than a tenth of the places for
-    // tiles stays empty in the rounds (10560 tiles in 3 x 256 units of 16: B =
-    // 24 51.4 and 55.6).
+    // activations (K 4096: 2049 tiles, B = 8 / 64 16.8 / 28.2 with two on four
+    // wavefronts, 18.9 / 31.4 with one on eight; 1800 tiles, B = 64 22.6 and
+    // 20.8), on eight wavefronts (3750 tiles: B = 64 36.7 on four, 33.5; 96
+    // FFN matrices: B = 32 470 and 453, B = 64 586 and 536), except up to 8
+    // tokens (24.2 and 24.6) and where more than a tenth of the places for
+    // tiles stays empty in the rounds (4800 tiles, B = 32 36.7 and 41.2; 10560
+    // tiles of a plan of K 2048 and 6016, B = 24 51.4 and 55.6; but 2300 to
+    // 3000 tiles, and 10560 of K 4096, run 5 to 9 % faster on eight).
     if (tiles > (int64_t)ncu * kMWide) {
       s.TM = 2;
       const int64_t places = (wide + ncu - 1) / ncu * ncu * (2 * kMWide);
